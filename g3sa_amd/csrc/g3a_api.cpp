@@ -48,7 +48,7 @@ struct DevBuf {
 // on a second one whose buffers are views into the device's static scratch
 // array.
 struct Work {
-  DevBuf lep_pool, eh_pool, tb_order, tb_ctr, tb_nw;
+  DevBuf eh_pool, tb_order, tb_ctr, tb_nw;
   DevBuf seed_key, seed_key2, seed_idx, seed_order, seed_sort_tmp;  // seeding order
   // seeding
   DevBuf intv, n_intv, n_seed, slow, intv_base, seed_off, counters, slow_list, slow_scratch, slow_n, slow_off;
@@ -106,7 +106,7 @@ struct g3a_ctx {
   int max_reads = 0;
   int64_t max_bases = 0;
   // index
-  DevBuf occ, pac, sa, ctg_off, ctg_len, ctg_alt, kmer, occn, sbc;
+  DevBuf occ, super, pac, sa, ctg_off, ctg_len, ctg_alt, kmer, occn, sbc;
   DevBuf ctg_names, ctg_name_off, log_tab;  // for the record formatter
   // batch text (names, qualities) and formatted records
   bool has_text = false;
@@ -120,9 +120,9 @@ struct g3a_ctx {
   bool has_input = false, has_output = false;
   DevBuf seq, off;
   int seed_ordered = 0;  // seed reads in minimizer order (1) or input order (0)
-  int seed_threads = 0, tb_threads = 0;  // resident maxima (the pools are sized for them)
+  int tb_threads = 0;  // resident maximum (the pool is sized for it)
   // k_seed grid: one 1024-thread block per compute unit keeps a single copy
-  // of the superblock counts in LDS and the rest for list entries
+  // of the superblock counts in LDS
   int seed_blocks_per_cu = 1;             // 0: the occupancy maximum
   int seed_block = 1024;                  // k_seed threads per block
   int chain_serial = 0;                   // chaining: 0 thread / wavefront tiers, 1 the B-tree code per read
@@ -136,7 +136,7 @@ struct g3a_ctx {
   DevBuf fmt_scan_tmp;            // scan storage of the formatter and output copy
   DevBuf pe_hist, pe_stat, pe_v, pe_out;  // paired-end statistics and pair choice
   // grids of the running call (sizes of the per-thread pools)
-  int run_seed_threads = 0, run_tb_threads = 0, run_lane_blocks = 0, run_slow_chunk = 16384;
+  int run_tb_threads = 0, run_lane_blocks = 0, run_slow_chunk = 16384;
   // batched-form extension
   int form = G3A_FORM_BATCHED;
   int n_cu = 0;
@@ -314,7 +314,7 @@ int init_runtime(g3a_ctx *ctx) {
 
 // The device index's buffers of a context (shared with its siblings).
 std::vector<DevBuf *> index_bufs(g3a_ctx *c) {
-  return {&c->occ,     &c->kmer,       &c->occn,    &c->sbc,     &c->pac,     &c->sa,       &c->ctg_off,
+  return {&c->occ,     &c->super,      &c->kmer,       &c->occn,    &c->sbc,     &c->pac,     &c->sa,       &c->ctg_off,
           &c->ctg_len, &c->ctg_alt,    &c->ctg_names, &c->ctg_name_off, &c->log_tab, &c->li_saf, &c->li_keys,
           &c->li_root, &c->li_leaf,    &c->li_knot, &c->li_leaf_a, &c->li_short, &c->li_ctr};
 }
@@ -470,7 +470,6 @@ int g3a_device_alloc_sibling(g3a_ctx *src, int max_reads, int64_t max_bases, g3a
   ctx->seed_block = src->seed_block;
   ctx->chain_serial = src->chain_serial;
   ctx->seed_ordered = src->seed_ordered;
-  ctx->seed_threads = src->seed_threads;
   ctx->tb_threads = src->tb_threads;
   ctx->use_graph = src->use_graph;
   std::memcpy(ctx->per_read, src->per_read, sizeof ctx->per_read);
@@ -493,16 +492,12 @@ int g3a_device_alloc_sibling(g3a_ctx *src, int max_reads, int64_t max_bases, g3a
 // allocation-free call no more seeding threads than reads, and smaller
 // traceback and extension grids, so that their per-thread pools fit the
 // scratch array.
-static void set_grids(g3a_ctx *ctx, int n, bool noalloc) {
-  if (!ctx->seed_threads) ctx->seed_threads = seed_grid_threads(ctx->n_cu, ctx->idx, ctx->seed_block);
+static void set_grids(g3a_ctx *ctx, bool noalloc) {
   if (!ctx->tb_threads) ctx->tb_threads = traceback_grid_threads(ctx->n_cu);
-  ctx->run_seed_threads = ctx->seed_threads;
   ctx->run_tb_threads = ctx->tb_threads;
   ctx->run_lane_blocks = ctx->n_cu * ctx->lane_blocks_per_cu;
   ctx->run_slow_chunk = 16384;
   if (noalloc) {
-    const int need = ((n + 127) / 128) * 128;
-    ctx->run_seed_threads = std::max(ctx->seed_block, std::min(ctx->seed_threads, need));
     ctx->run_tb_threads = std::min(ctx->tb_threads, 4096);
     ctx->run_lane_blocks = std::min(ctx->run_lane_blocks, 64);
     ctx->run_slow_chunk = 16;
@@ -526,7 +521,7 @@ static int alloc_reads(g3a_ctx *ctx, int n) {
       ensure(ctx, ctx->w->seed_idx, (size_t)n * 4 + 4) || ensure(ctx, ctx->w->seed_order, (size_t)n * 4 + 4) ||
       ensure(ctx, ctx->w->seed_sort_tmp, seed_sort_tmp_bytes(n)))
     return G3A_E_HIP;
-  return ensure(ctx, ctx->w->lep_pool, (size_t)ctx->run_seed_threads * (kLepCap + kFoundCap) * sizeof(Intv));
+  return 0;
 }
 
 static int alloc_seeds(g3a_ctx *ctx, int64_t T_s, int n) {
@@ -560,11 +555,11 @@ static int alloc_paths(g3a_ctx *ctx, int64_t T_z, int64_t T_c) {
 // Set-up sizes for a batch of max_reads reads and max_bases bases: 12 seeds,
 // 4 extension tasks and one alignment per read, direction bytes for
 // 4 x max_bases and the CIGAR capacity of one alignment per read.
-static void set_grids(g3a_ctx *ctx, int n, bool noalloc);
+static void set_grids(g3a_ctx *ctx, bool noalloc);
 
 static int reserve_workspace(g3a_ctx *ctx) {
   const int n = ctx->max_reads;
-  set_grids(ctx, n, false);
+  set_grids(ctx, false);
   const int64_t nb = ctx->max_bases;
   if (alloc_reads(ctx, n) || alloc_seeds(ctx, 12 * (int64_t)n, n) || alloc_tasks(ctx, 4 * (int64_t)n) ||
       alloc_alns(ctx, n) || alloc_paths(ctx, 4 * nb, 4 * nb + 4 * (int64_t)n))
@@ -615,6 +610,8 @@ int g3a_memcpy_index(g3a_ctx *ctx) {
       if ((sb << 32) < rows) bwa_occ_rows(h.bwt_words.data(), h.primary, sb << 32, c);
       for (int k = 0; k < 4; ++k) x.super[sb][k] = (int64_t)c[k];
     }
+    if (ensure(ctx, ctx->super, sizeof x.super)) return G3A_E_HIP;
+    HIPCK(hipMemcpy(ctx->super.p, x.super, sizeof x.super, hipMemcpyHostToDevice));
   }
   // 16 zero bytes of padding: word-wise readers may read past the last base
   if (ensure(ctx, ctx->pac, h.pac.size() + 16)) return G3A_E_HIP;
@@ -648,6 +645,7 @@ int g3a_memcpy_index(g3a_ctx *ctx) {
     HIPCK(hipMemcpy(ctx->log_tab.p, lt.data(), lt.size() * 4, hipMemcpyHostToDevice));
   }
   x.occ = P<uint32_t>(ctx->occ);
+  x.super_dev = P<int64_t>(ctx->super);
   build_counts(h, x.count);
   x.primary = (int64_t)h.primary;
   x.n = (int64_t)h.seq_len;
@@ -660,17 +658,23 @@ int g3a_memcpy_index(g3a_ctx *ctx) {
   x.ctg_off = P<int64_t>(ctx->ctg_off);
   x.ctg_len = P<int64_t>(ctx->ctg_len);
   x.ctg_alt = P<int32_t>(ctx->ctg_alt);
+  // the interval of every kKmer-mer: 32-bit fields, or 64-bit ones in the
+  // wide layout
   x.kmer = nullptr;
+  x.kmer64 = nullptr;
   x.occn = x.sbc = nullptr;
-  if (narrow) {  // 32-bit interval fields
+  if (ensure(ctx, ctx->kmer, ((size_t)3 << (2 * kKmer)) * (narrow ? 4 : 8))) return G3A_E_HIP;
+  if (narrow) {
     x.occn = P<uint32_t>(ctx->occn);
     x.sbc = P<uint32_t>(ctx->sbc);
-    if (ensure(ctx, ctx->kmer, ((size_t)3 << (2 * kKmer)) * 4)) return G3A_E_HIP;
     launch_kmer_table(x, P<uint32_t>(ctx->kmer), ctx->stream);
-    HIPCK(hipStreamSynchronize(ctx->stream));
-    HIPCK(hipGetLastError());
-    x.kmer = P<uint32_t>(ctx->kmer);
+  } else {
+    launch_kmer_table64(x, P<int64_t>(ctx->kmer), ctx->stream);
   }
+  HIPCK(hipStreamSynchronize(ctx->stream));
+  HIPCK(hipGetLastError());
+  if (narrow) x.kmer = P<uint32_t>(ctx->kmer);
+  else x.kmer64 = P<int64_t>(ctx->kmer);
   if (int rc = reserve_workspace(ctx)) return rc;
   ctx->index_on_device = true;
   return G3A_OK;
@@ -924,7 +928,6 @@ static int enqueue_batch(g3a_ctx *ctx, int n, const Caps &c, bool timed) {
   sa.n_seed = P<int64_t>(w.n_seed);
   sa.slow = P<int32_t>(w.slow);
   sa.fm_steps = cnt + 0;
-  sa.lep_pool = P<Intv>(w.lep_pool);
   sa.li_stats = ctx->idx.saf ? cnt + 32 : nullptr;
   sa.next_read = P<int32_t>(w.counters) + kNextReadSlot32;
   sa.order = nullptr;
@@ -936,11 +939,7 @@ static int enqueue_batch(g3a_ctx *ctx, int n, const Caps &c, bool timed) {
     sa.order = P<int32_t>(w.seed_order);
   }
   if (timed) HIPCK(hipEventRecord(ctx->kev[0], s));
-  const int seed_run =
-      ctx->seed_blocks_per_cu > 0 && ctx->seed_blocks_per_cu * ctx->seed_block * ctx->n_cu < ctx->run_seed_threads
-          ? ctx->seed_blocks_per_cu * ctx->seed_block * ctx->n_cu
-          : ctx->run_seed_threads;
-  launch_seed(sa, seed_run, ctx->seed_blocks_per_cu, ctx->seed_block, s);
+  launch_seed(sa, ctx->n_cu, ctx->seed_blocks_per_cu, ctx->seed_block, s);
   if (timed) HIPCK(hipEventRecord(ctx->kev[1], s));
   ctx->kev_used[0] = timed;
   launch_collect_slow(n, P<int32_t>(w.slow), P<int32_t>(w.slow_list), n_slow_dev, P<int64_t>(w.intv_base), kSlotCap, s);
@@ -1093,7 +1092,7 @@ static std::string graph_key(const g3a_ctx *ctx, int n, const Caps &c) {
   put(&ctx->idx, sizeof ctx->idx);
   put(&ctx->opt, sizeof ctx->opt);
   const int v[] = {ctx->form, ctx->strip_rows, ctx->lane_blocks_per_cu, ctx->wave_blocks_per_cu, ctx->ext_packed,
-                   ctx->seed_blocks_per_cu, ctx->seed_block, ctx->run_seed_threads, ctx->run_tb_threads, ctx->run_lane_blocks,
+                   ctx->seed_blocks_per_cu, ctx->seed_block, ctx->run_tb_threads, ctx->run_lane_blocks,
                    ctx->run_slow_chunk, ctx->chain_serial};
   put(v, sizeof v);
   put(&ctx->buf_gen, sizeof ctx->buf_gen);
@@ -1219,7 +1218,7 @@ int g3a_bwa_align(g3a_ctx *ctx) {
   if (!ctx->index_on_device || !ctx->has_input) return fail(ctx, G3A_E_STATE, "index or input not on device");
   HIPCK(hipSetDevice(ctx->device));
   ctx->w = &ctx->own;
-  set_grids(ctx, ctx->n_reads, false);
+  set_grids(ctx, false);
   return align_batch(ctx);
 }
 
@@ -1239,7 +1238,7 @@ int g3a_bwa_align_noalloc(g3a_ctx *ctx) {
   ctx->scratch_work = Work{};
   ctx->w = &ctx->scratch_work;
   ctx->arena = &arena;
-  set_grids(ctx, ctx->n_reads, true);
+  set_grids(ctx, true);
   const int rc = align_batch(ctx);
   ctx->arena = nullptr;
   if (rc) ctx->has_output = false;
@@ -1565,10 +1564,7 @@ int g3a_set_seed_grid(g3a_ctx *ctx, int threads_per_block, int blocks_per_cu) {
   if (!ctx || blocks_per_cu < 0 || blocks_per_cu > 64 || threads_per_block < 64 || threads_per_block > 1024 ||
       threads_per_block % 64)
     return G3A_E_ARG;
-  if (threads_per_block != ctx->seed_block) {
-    ctx->seed_block = threads_per_block;
-    ctx->seed_threads = 0;  // the resident maximum (and the list pool) follow the block size
-  }
+  ctx->seed_block = threads_per_block;
   ctx->seed_blocks_per_cu = blocks_per_cu;
   return G3A_OK;
 }
@@ -1844,7 +1840,7 @@ void g3a_destroy(g3a_ctx *ctx) {
   hipSetDevice(ctx->device);
   if (ctx->stream) hipStreamSynchronize(ctx->stream);
   free_graph(ctx);
-  DevBuf *bufs[] = {&ctx->occ, &ctx->kmer, &ctx->occn, &ctx->sbc, &ctx->pac, &ctx->sa, &ctx->ctg_off, &ctx->ctg_len, &ctx->ctg_alt, &ctx->seq, &ctx->off,
+  DevBuf *bufs[] = {&ctx->occ, &ctx->super, &ctx->kmer, &ctx->occn, &ctx->sbc, &ctx->pac, &ctx->sa, &ctx->ctg_off, &ctx->ctg_len, &ctx->ctg_alt, &ctx->seq, &ctx->off,
                     &ctx->own.intv, &ctx->own.n_intv, &ctx->own.n_seed, &ctx->own.slow, &ctx->own.intv_base, &ctx->own.seed_off,
                     &ctx->own.counters, &ctx->own.slow_list, &ctx->own.slow_scratch, &ctx->own.slow_n, &ctx->own.slow_off, &ctx->own.seeds,
                     &ctx->own.seeds2, &ctx->own.ch, &ctx->own.nxt, &ctx->own.order, &ctx->own.tmpi, &ctx->own.w16, &ctx->own.kept, &ctx->own.nodes,
@@ -1855,7 +1851,7 @@ void g3a_destroy(g3a_ctx *ctx) {
                     &ctx->own.seed_order, &ctx->own.seed_sort_tmp,
                     &ctx->own.ext_res[0], &ctx->own.ext_res[1], &ctx->own.ext_key, &ctx->own.ext_hist, &ctx->own.totals,
                     &ctx->own.ext_sorted, &ctx->own.ext_slow, &ctx->own.ext_ctr, &ctx->own.ext_rowbuf,
-                    &ctx->own.lep_pool, &ctx->own.eh_pool, &ctx->own.tb_order, &ctx->own.tb_ctr, &ctx->own.tb_nw, &ctx->li_saf, &ctx->li_keys,
+                    &ctx->own.eh_pool, &ctx->own.tb_order, &ctx->own.tb_ctr, &ctx->own.tb_nw, &ctx->li_saf, &ctx->li_keys,
                     &ctx->li_root, &ctx->li_leaf, &ctx->li_knot, &ctx->li_leaf_a, &ctx->li_short, &ctx->li_ctr,
                     &ctx->ctg_names, &ctx->ctg_name_off, &ctx->log_tab, &ctx->names, &ctx->name_off, &ctx->quals,
                     &ctx->qual_off, &ctx->txt_len, &ctx->txt_off, &ctx->txt, &ctx->txt_bound, &ctx->stage_off, &ctx->txt_stage, &ctx->fmt_flag, &ctx->mapq, &ctx->md_len,

@@ -73,6 +73,7 @@ struct alignas(16) LiKnot {
 struct DevIndex {
   const uint32_t *occ;
   int64_t super[4][4];
+  const int64_t *super_dev;  // the same 16 values in device memory (host code reads super)
   int64_t count[5];  // count[c] = 1 + #bases < c (the '$' row first), count[4] = n+1
   int64_t primary;   // row whose suffix starts at text position 0 (BWT '$')
   int64_t n;         // text length 2*l_pac; rows 0..n
@@ -86,8 +87,10 @@ struct DevIndex {
   const int64_t *ctg_len;
   const int32_t *ctg_alt;
   // bidirectional interval (k, l, s) of every kKmer-mer, 2-bit code of the
-  // first base highest; null when the text has 2^32 rows or more
+  // first base highest: 32-bit fields for the narrow layout, 64-bit ones for
+  // the wide one (the other is null)
   const uint32_t *kmer;
+  const int64_t *kmer64;
   // texts of fewer than 2^32 rows: 16-byte lines of 32 rows (21-bit counts
   // of bases 0-2 relative to a 2^21-row superblock, then 32 symbols) and the
   // superblocks' four absolute counts (uint32 each); null otherwise
@@ -134,7 +137,8 @@ G3A_HD IntvT<Q> intv_cast(const IntvT<P> &a) {
 // kernel argument) a per-lane c would otherwise turn into a memory load
 template <class T>
 G3A_HD T pick4(const T *v, int c) {
-  return c == 0 ? v[0] : c == 1 ? v[1] : c == 2 ? v[2] : v[3];
+  const T a = v[0], b = v[1], d = v[2], e = v[3];
+  return c == 0 ? a : c == 1 ? b : c == 2 ? d : e;
 }
 
 struct Seed {
@@ -262,14 +266,23 @@ G3A_HD OccLine occ_line(const DevIndex &x, int64_t line) {
   L.w1 = (uint64_t)b[6] | (uint64_t)b[7] << 32;
   return L;
 }
+// Count of base c in the rows before 2^32-row superblock sb.  On the device a
+// load: super is a kernel argument, and indexing it would copy the arguments
+// to scratch memory.
+G3A_HD int64_t super_count(const DevIndex &x, int sb, int c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return x.super_dev[(sb << 2) + c];
+#else
+  return x.super[sb][c];
+#endif
+}
 // Occ(p, c) for all c from p's line
 G3A_HD void occ_at(const DevIndex &x, const OccLine &L, int64_t p, int64_t o[4]) {
   uint32_t in[4];
   line_counts(L.w0, L.w1, (int)(p & 63), in);
-  const int64_t *sb = x.super[p >> 32];
   const int dollar = (p >> 6) == (x.primary >> 6) && p >= x.primary;
 #pragma unroll
-  for (int c = 0; c < 4; ++c) o[c] = sb[c] + (int64_t)L.c[c] + in[c];
+  for (int c = 0; c < 4; ++c) o[c] = super_count(x, (int)(p >> 32), c) + (int64_t)L.c[c] + in[c];
   o[0] -= dollar;
 }
 
@@ -343,12 +356,6 @@ G3A_HD void occ4_pair(const DevIndex &x, uint32_t p1, uint32_t p2, uint32_t o1[4
   occ_at(x, L2, p2, o2);
 }
 
-G3A_HD int64_t occ1(const DevIndex &x, int64_t p, int c) {
-  int64_t o[4];
-  occ4(x, p, o);
-  return o[c];
-}
-
 // BWT character of row k (4 for the '$' row)
 G3A_HD int bwt_char(const DevIndex &x, int64_t k) {
   if (k == x.primary) return 4;
@@ -384,32 +391,29 @@ G3A_HD void backward_ext(const DevIndex &x, const IntvT<P> &in, int base, IntvT<
   out.s = pick4(s, base);
 }
 
-// Occ(p, c) of one base c from p's narrow line: one popcount of the rows
-// [line start, p] holding c ('$' is stored as 0 and not counted)
+// Rows of one base c (0..3) among the symbols of w selected by m (the even
+// bits of their pairs): one popcount, no branch on c
+G3A_HD uint32_t sym_count(uint64_t w, uint64_t m, int c) {
+  const uint64_t d = w ^ (0x5555555555555555ULL * (uint64_t)c);  // symbols equal to c become 00
+  return (uint32_t)G3A_POPC(~(d | d >> 1) & m);
+}
+// Occ(p, c) of one base c from p's narrow line ('$' is stored as 0 and not
+// counted)
 G3A_HD uint32_t occ1_at(const DevIndex &x, const OccLineN &L, uint32_t p, int c) {
-  const int y = (int)(p & 31);
-  const uint64_t m = (~0ULL << (62 - 2 * y)) & 0x5555555555555555ULL;
-  const uint64_t hi = (L.w >> 1) & m, lo = L.w & m;
-  const uint64_t sel = c == 3 ? hi & lo : c == 2 ? hi & ~lo : c == 1 ? lo & ~hi : m & ~hi & ~lo;
-  const uint32_t n = (uint32_t)G3A_POPC(sel);
-  uint32_t sc;
-#if defined(__HIP_DEVICE_COMPILE__)
-  const uint4 sb = *(const uint4 *)(x.sbc + ((p >> 21) << 2));
-  sc = c == 0 ? sb.x : c == 1 ? sb.y : c == 2 ? sb.z : sb.w;
-#else
-  sc = x.sbc[((p >> 21) << 2) + c];
-#endif
-  const uint32_t r0 = (uint32_t)(L.cnt & 0x1fffff), r1 = (uint32_t)(L.cnt >> 21) & 0x1fffff,
-                 r2 = (uint32_t)(L.cnt >> 42) & 0x1fffff;
+  const uint32_t y = p & 31;
+  const uint32_t n = sym_count(L.w, (~0ULL << (62 - 2 * y)) & 0x5555555555555555ULL, c);
+  const uint32_t sc = x.sbc[((p >> 21) << 2) + (uint32_t)c];
   const uint32_t pr = (uint32_t)x.primary, ls = p & ~31u, ss = p & ~((1u << 21) - 1);
   const uint32_t dol_before = pr >= ss && pr < ls, dol_in = pr >= ls && pr <= p;
-  const uint32_t rc = c == 0 ? r0 : c == 1 ? r1 : c == 2 ? r2 : (ls - ss) - r0 - r1 - r2 - dol_before;
-  return sc + rc + n - (c == 0 ? dol_in : 0u);
+  const uint32_t r3 = (ls - ss) - (uint32_t)(L.cnt & 0x1fffff) - ((uint32_t)(L.cnt >> 21) & 0x1fffff) -
+                      ((uint32_t)(L.cnt >> 42) & 0x1fffff) - dol_before;
+  const uint32_t rc = (uint32_t)(L.cnt >> (c == 3 ? 0 : 21 * c)) & 0x1fffff;
+  return sc + (c == 3 ? r3 : rc) + n - (c == 0 ? dol_in : 0u);
 }
 
 // Backward extension by `base` of k and s only (l is left as it was): for
 // the backward phases, whose intervals are only extended backward again or
-// output, and neither reads l.  Narrow layout: one base's count per row.
+// output, and neither reads l.  One base's count per row.
 G3A_HD void backward_ext_ks(const DevIndex &x, const IntvT<uint32_t> &in, int base, IntvT<uint32_t> &out) {
   const uint32_t p1 = in.k - 1, p2 = in.k + in.s - 1;
   const OccLineN L1 = occn_line(x, p1 >> 5), L2 = occn_line(x, p2 >> 5);  // overlapping fetches
@@ -419,8 +423,42 @@ G3A_HD void backward_ext_ks(const DevIndex &x, const IntvT<uint32_t> &in, int ba
   out.l = in.l;
   out.s = b - a;
 }
+// The same in the wide layout: base c's count and the two symbol words of a line
+struct OccLine1 {
+  uint32_t cnt;
+  uint64_t w0, w1;
+};
+G3A_HD OccLine1 occ_line1(const DevIndex &x, int64_t line, int c) {
+  const uint32_t *b = x.occ + (line << 3);
+  OccLine1 L;
+  L.cnt = b[c];
+#if defined(__HIP_DEVICE_COMPILE__)
+  const uint4 v = *(const uint4 *)(b + 4);
+  L.w0 = (uint64_t)v.x | (uint64_t)v.y << 32;
+  L.w1 = (uint64_t)v.z | (uint64_t)v.w << 32;
+#else
+  L.w0 = (uint64_t)b[4] | (uint64_t)b[5] << 32;
+  L.w1 = (uint64_t)b[6] | (uint64_t)b[7] << 32;
+#endif
+  return L;
+}
+G3A_HD int64_t occ1_at(const DevIndex &x, const OccLine1 &L, int64_t p, int c) {
+  const uint64_t E = 0x5555555555555555ULL;
+  const int y = (int)(p & 63);
+  const uint64_t m = (~0ULL << (62 - 2 * (y & 31))) & E, m0 = y < 32 ? m : E, m1 = y < 32 ? 0 : m;
+  const int dollar = (p >> 6) == (x.primary >> 6) && p >= x.primary;
+  return super_count(x, (int)(p >> 32), c) + (int64_t)L.cnt + sym_count(L.w0, m0, c) + sym_count(L.w1, m1, c) -
+         (c == 0 ? dollar : 0);
+}
+G3A_HD int64_t occ1(const DevIndex &x, int64_t p, int c) { return occ1_at(x, occ_line1(x, p >> 6, c), p, c); }
 G3A_HD void backward_ext_ks(const DevIndex &x, const IntvT<int64_t> &in, int base, IntvT<int64_t> &out) {
-  backward_ext(x, in, base, out);
+  const int64_t p1 = in.k - 1, p2 = in.k + in.s - 1;
+  const OccLine1 L1 = occ_line1(x, p1 >> 6, base), L2 = occ_line1(x, p2 >> 6, base);  // overlapping fetches
+  const int64_t a = occ1_at(x, L1, p1, base);
+  const int64_t b = occ1_at(x, L2, p2, base);
+  out.k = pick4(x.count, base) + a;
+  out.l = in.l;
+  out.s = b - a;
 }
 
 // backwardExtBackward (fmindex.cu:162-180): k and s only
@@ -450,7 +488,7 @@ G3A_HD int64_t sa_value(const DevIndex &x, int64_t k, int64_t *steps) {
   while (k & mask) {
     if (k == x.primary) return t;
     int c = bwt_char(x, k);
-    k = x.count[c] - 1 + occ1(x, k, c);
+    k = pick4(x.count, c) - 1 + occ1(x, k, c);
     ++t;
   }
   if (steps) *steps += t;
@@ -1323,14 +1361,16 @@ G3A_HD void reseed_round3(const DevIndex &x, const Opt &o, const uint8_t *q, int
 }
 
 // Interval of k-mer `code` (kKmer bases, first base in the highest bits) by
-// kKmer-1 forward steps from the first base: the k-mer table's entries.
-G3A_HD void kmer_interval(const DevIndex &x, uint32_t code, uint32_t out[3]) {
+// kKmer-1 forward steps from the first base: the k-mer table's entries, of
+// 32-bit fields (narrow layout) or 64-bit ones (wide).
+template <class T>
+G3A_HD void kmer_interval(const DevIndex &x, uint32_t code, T out[3]) {
   Intv seed;
   intv_init(x, seed, (int)(code >> (2 * (kKmer - 1))) & 3);
   for (int i = kKmer - 2; i >= 0; --i) forward_ext(x, seed, (int)(code >> (2 * i)) & 3);
-  out[0] = (uint32_t)seed.k;
-  out[1] = (uint32_t)seed.l;
-  out[2] = (uint32_t)seed.s;
+  out[0] = (T)seed.k;
+  out[1] = (T)seed.l;
+  out[2] = (T)seed.s;
 }
 
 // ---------------------------------------------------------------------------

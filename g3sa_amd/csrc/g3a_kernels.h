@@ -8,11 +8,10 @@
 
 namespace g3a {
 
-constexpr int kSlowLep = 400;                  // slow-path LEP list capacity
-constexpr int kSlowScratch = 5 * kSlowLep;     // Intv entries of scratch per slow read
+constexpr int kSlowScratch = 800;              // Intv entries of scratch per slow read
 constexpr int kSlotCap = 64;                   // fast-path interval slots per read
-constexpr int kLepCap = 64;                    // fast-path LEP list capacity
-constexpr int kFoundCap = 16;                  // fast-path found-match (and reseed seed) list capacity
+constexpr int kLepCap = 64;                    // fast-path list capacity
+constexpr int kFoundCap = 16;                  // fast-path capacity of one search's found matches
 
 struct SeedArgs {
   const int32_t *stop;  // when *stop is set the kernel returns at once (null: never)
@@ -27,11 +26,9 @@ struct SeedArgs {
   int64_t *n_seed;
   int32_t *slow;
   int64_t *fm_steps;
-  Intv *lep_pool;    // kLepCap + kFoundCap entries per k_seed thread
   const int32_t *order;  // reads in processing order, or null for input order
-  int lep_lds;           // LEP entries per thread kept in LDS (narrow form; set by launch_seed)
   int64_t *li_stats;     // learned-index form counters (6), or null
-  int32_t *next_read;    // zeroed before k_seed: reads are handed out by an atomic counter (null: fixed stride)
+  int32_t *next_read;    // zeroed before k_seed, which hands the reads out by it
 };
 
 // Counts known only on the device (totals of a batch's seeds, tasks and
@@ -176,12 +173,10 @@ struct TbArgs {
   int32_t *tb_nw;     // n_alns: global-alignment scores from k_tb_wave_dp
 };
 
-// threads of k_seed's persistent grid in blocks of `block` threads
-// (occupancy-limited, n_cu compute units)
-int seed_grid_threads(int n_cu, const DevIndex &x, int block);
-// blocks_per_cu: the grid the caller runs (0: the occupancy maximum), which
-// with the block size sets the LDS share of each block for the LEP lists
-void launch_seed(const SeedArgs &a, int n_threads, int blocks_per_cu, int block, hipStream_t s);
+// k_seed's persistent grid: blocks of at most `block` threads, blocks_per_cu
+// of them on each of n_cu compute units (0, or more than fit: the occupancy
+// maximum)
+void launch_seed(const SeedArgs &a, int n_cu, int blocks_per_cu, int block, hipStream_t s);
 // slow reads list[0, n_list) of the whole list's *n_dev (from entry c0 of it)
 void launch_seed_slow(const SeedArgs &a, const int32_t *list, int n_list, const int32_t *n_dev, int c0, Intv *scratch,
                       const int64_t *pool_off, Intv *pool, int pass, int from_scratch, hipStream_t s);
@@ -196,8 +191,10 @@ void launch_ext_wave(const ExtSideArgs &a, int n_blocks, hipStream_t s);
 void launch_ext_finish(const ExtFinishArgs &a, hipStream_t s);
 void launch_fill_i32(int32_t *p, int n, int32_t v, hipStream_t s);
 void launch_clamp_codes(uint8_t *seq, int64_t n, hipStream_t s);
-// fills the 3 * 4^kKmer words of the k-mer interval table
+// fills the 3 * 4^kKmer words of the k-mer interval table of the narrow, or
+// the wide layout
 void launch_kmer_table(const DevIndex &x, uint32_t *table, hipStream_t s);
+void launch_kmer_table64(const DevIndex &x, int64_t *table, hipStream_t s);
 // record formatting (g3a_text.hip): per-read text lengths, then the text at
 // txt_off; per-alignment MAPQ and MD-string lengths, then the MD strings
 // the batch's records: each read's text length (write = false: len), or

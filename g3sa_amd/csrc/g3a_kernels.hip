@@ -1,9 +1,7 @@
-// HIP kernels of the BWA-MEM hot path for MI355X (gfx950, wave64).
+// HIP kernels of the BWA-MEM hot path for MI355X (gfx950, wave64); seeding is
+// in g3a_seed.hip.
 //
 // Stage kernels (one launch each, all on the context's stream):
-//   k_seed           thread per read: SMEM + reseed + third-round intervals
-//   k_seed_slow      wavefront per read, for reads whose lists outgrew the
-//                    fast path's buffers (LDS lists, list entries on lanes)
 //   k_sa_lookup      thread per seed: SA interval row -> reference position
 //   k_chain          wavefront per read: seed sort, chaining, chain filter,
 //                    tasks (lane 0 in global memory for the rare large read)
@@ -71,114 +69,12 @@ __device__ __forceinline__ T gather(const T (&v)[NC], int e) {  // e per lane; c
   }
   return x;
 }
-// The next item of a work counter for each active lane: one atomic per
-// wavefront, its active lanes taking consecutive items.
-__device__ __forceinline__ int wave_next(int32_t *ctr) {
-  const uint64_t m = __ballot(true);
-  const int leader = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)m) - 1);
-  int base = 0;
-  if ((int)(threadIdx.x & 63) == leader) base = atomicAdd(ctr, __popcll(m));
-  base = __builtin_amdgcn_readlane(base, leader);
-  return base + __popcll(m & ((1ull << (threadIdx.x & 63)) - 1));
-}
 __device__ __forceinline__ void wave_lds_sync() {  // this wavefront's LDS stores are seen by its lanes
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-
-// ---------------------------------------------------------------------------
-// seeding
-// ---------------------------------------------------------------------------
-// Persistent grid: each thread takes the next read from a device counter
-// (one atomic per wavefront and turn, its active lanes taking consecutive
-// reads), so that a thread held up by a long read takes fewer
-// (r = tid, tid + T, ... when no counter is given).  Its LEP
-// lists live in a global pool slice of its own, contiguous per thread (a
-// divergent list access then touches one cache line; private memory would
-// scatter every entry over eight lines of the per-lane swizzle).
-// In the narrow form the superblock counts (16 B per 2^21 rows, at most
-// 32 KB) are copied to LDS, so an Occ lookup costs one 16-byte global load,
-// and the first a.lep_lds entries of each thread's LEP list live in LDS
-// after them (12 B per entry, lanes interleaved), the rest in the thread's
-// global slice: the list traffic then stays out of the caches that the Occ
-// lines need.
-template <bool L, class B>
-__device__ __forceinline__ void seed_reads(SeedArgs &a, B &buf, int gtid, int nthreads) {
-  using I = typename B::I;
-  int64_t steps = 0;
-  // learned-index form: range lookups, lookups answered by the FM-index,
-  // text runs, run bases, lookups the model narrowed, model windows missed
-  int64_t lc[6] = {0, 0, 0, 0, 0, 0};
-  for (int i = a.next_read ? wave_next(a.next_read) : gtid; i < a.n_reads;
-       i = a.next_read ? wave_next(a.next_read) : i + nthreads) {
-    const int r = a.order ? a.order[i] : i;
-    const int off = a.off[r], len = a.off[r + 1] - off;
-    const uint8_t *q = a.seq + off;
-    IntvSink sink{a.intv + (int64_t)r * a.slot_cap, a.slot_cap, 0, 0, a.opt.max_occ};
-    if (len > kMaxReadLen) {  // unaligned (documented limit)
-      a.n_intv[r] = 0;
-      a.n_seed[r] = 0;
-      a.slow[r] = 0;
-      continue;
-    }
-    bool ok = smem_round1<L>(a.idx, a.opt, q, len, sink, buf, &steps, lc);
-    if (ok) {
-      const int nsm = sink.n < sink.cap ? sink.n : sink.cap;
-      if (sink.n <= sink.cap) {
-        for (int k = 0; ok && k < nsm; ++k) {
-          Intv smem = sink.slot[k];
-          ok = reseed_one(a.idx, a.opt, q, len, smem, buf.a, buf.f, buf.cap, buf.cap_f, sink, &steps);
-        }
-      } else ok = false;
-      if (ok) reseed_round3<decltype(I::s), L>(a.idx, a.opt, q, len, sink, &steps, lc);
-    }
-    ok = ok && sink.n <= sink.cap;
-    a.slow[r] = ok ? 0 : 1;
-    a.n_intv[r] = ok ? sink.n : 0;
-    a.n_seed[r] = ok ? sink.n_seed : 0;
-  }
-  if (a.fm_steps) {  // one atomic per wavefront
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) steps += __shfl_xor(steps, o);
-    if ((threadIdx.x & 63) == 0 && steps) atomicAdd((unsigned long long *)a.fm_steps, (unsigned long long)steps);
-  }
-  if (L && a.li_stats) {
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-      int64_t v = lc[k];
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
-      if ((threadIdx.x & 63) == 0 && v) atomicAdd((unsigned long long *)a.li_stats + k, (unsigned long long)v);
-    }
-  }
-}
-
-// L: the learned-index form (text comparison of unique matches, the
-// model's intervals in the last round); a separate kernel, so that the
-// FM-only one keeps its register budget
-template <class E, bool L>
-__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(L ? 5 : 4))) k_seed(SeedArgs a) {
-  extern __shared__ uint4 sb_lds[];
-  const int gtid = blockIdx.x * blockDim.x + threadIdx.x;
-  const int nthreads = gridDim.x * blockDim.x;
-  E *la = reinterpret_cast<E *>(a.lep_pool) + (size_t)gtid * (kLepCap + kFoundCap), *lf = la + kLepCap;
-  if constexpr (E::kNarrow) {
-    const int n_sb = (int)(((uint64_t)a.idx.n + 1) >> 21) + 1;
-    const uint4 *src = (const uint4 *)a.idx.sbc;
-    for (int k = threadIdx.x; k < n_sb; k += blockDim.x) sb_lds[k] = src[k];
-    __syncthreads();
-    a.idx.sbc = (const uint32_t *)sb_lds;
-    LepBuf<SplitList, GlobalList<E>> buf{
-        SplitList{(uint32_t *)(sb_lds + n_sb) + threadIdx.x, (int)blockDim.x, a.lep_lds, la}, GlobalList<E>{lf},
-        kLepCap, kFoundCap};
-    seed_reads<L>(a, buf, gtid, nthreads);
-  } else {
-    GlobalBuf<E> buf{GlobalList<E>{la}, GlobalList<E>{lf}, kLepCap, kFoundCap};
-    seed_reads<false>(a, buf, gtid, nthreads);
-  }
-}
 
 // Seeding order.  Overlapping reads of one locus walk the FM-index through
 // the same intervals; given neighbouring lanes, their Occ lines are still in
@@ -216,198 +112,6 @@ __global__ void __launch_bounds__(256) k_seed_keys(const uint8_t *seq, const int
   }
   key[r] = best >> 8;  // 24-bit key, sorted on bits [0, 24)
   idx[r] = r;
-}
-
-// The backward steps of rounds 1 and 2 on a wavefront: entry j on lane
-// j % 64 of chunk j / 64 extends in parallel with the others, then one pass
-// in list order over the lanes' results takes the decisions that depend on
-// the entries before (which entries go on, the new start, the seed), and the
-// entries that go on are written back in order.  The lists are in LDS and
-// every lane sees the same list; the results equal SerialBack's.
-struct WaveBack {
-  static constexpr int kChunks = (kMaxReadLen + 63) / 64;  // no list of a read holds more entries
-  template <class L, class LF>
-  static __device__ int round1(const DevIndex &x, const Opt &o, const L &list, int np, int i, int c, const LF &fl,
-                               int &nf, int cap, int cap_f, int &last_start, int64_t *) {
-    using I = typename L::I;
-    const int lane = threadIdx.x & 63;
-    I ok[kChunks];
-    int pm[kChunks], pn[kChunks];
-    uint64_t ext[kChunks], fail[kChunks];
-    if (np > 64 * kChunks) return -1;  // (no read of <= kMaxReadLen bases gets here)
-    wave_lds_sync();
-#pragma unroll
-    for (int k = 0; k < kChunks; ++k) {
-      const int j = 64 * k + lane;
-      const bool live = j < np;
-      bool e = false;
-      pm[k] = pn[k] = 0;
-      if (live) {
-        const I pj = list.get(j);
-        pm[k] = pj.m;
-        pn[k] = pj.n;
-        if (c >= 0) {
-          backward_ext_ks(x, pj, c, ok[k]);
-          e = ok[k].s >= 1;
-        }
-      }
-      ext[k] = __ballot(live && e);
-      fail[k] = __ballot(live && !e);
-    }
-    int first_ext = np, first_fail = np;
-#pragma unroll
-    for (int k = kChunks - 1; k >= 0; --k) {
-      if (ext[k]) first_ext = 64 * k + __ffsll((unsigned long long)ext[k]) - 1;
-      if (fail[k]) first_fail = 64 * k + __ffsll((unsigned long long)fail[k]) - 1;
-    }
-    // a new start: the first entry that does not extend, none before it did
-    if (first_fail < first_ext && i + 1 < last_start) {
-      last_start = i + 1;
-      I p = list.get(first_fail);
-      if (p.n - i >= o.min_seed_len) {
-        p.m = i + 1;
-        if (nf == cap_f) return -1;
-        fl.put(nf++, p);  // every lane stores the same entry
-      }
-    }
-    // the entries that go on: each extension whose size differs from the
-    // last one kept
-    uint64_t keep[kChunks];
-    int nc = 0;
-    decltype(I::s) last_s = 0;
-#pragma unroll
-    for (int k = 0; k < kChunks; ++k) {
-      keep[k] = 0;
-      for (uint64_t m = ext[k]; m; m &= m - 1) {
-        const int b = __ffsll((unsigned long long)m) - 1;
-        const auto sb = lane_read(ok[k].s, b);
-        if (nc == 0 || sb != last_s) {
-          keep[k] |= 1ull << b;
-          ++nc;
-          last_s = sb;
-        }
-      }
-    }
-    if (nc > cap) return -1;
-    wave_lds_sync();  // every entry was read above
-    int before = 0;
-#pragma unroll
-    for (int k = 0; k < kChunks; ++k) {
-      if ((keep[k] >> lane) & 1) {
-        I e = ok[k];
-        e.m = pm[k];
-        e.n = pn[k];
-        list.put(before + __popcll(keep[k] & ((1ull << lane) - 1)), e);
-      }
-      before += __popcll(keep[k]);
-    }
-    wave_lds_sync();
-    return nc;
-  }
-  template <class L, class LF, class P>
-  static __device__ int reseed(const DevIndex &x, const Opt &o, const L &leps, int num_old, int m, int base,
-                               P min_seed_intv, const LF &seeds, int &ns, int cap_s, int64_t *) {
-    using I = typename L::I;
-    const int lane = threadIdx.x & 63;
-    I ex[kChunks];
-    int ln[kChunks];
-    if (num_old > 64 * kChunks) return -1;  // (no read of <= kMaxReadLen bases gets here)
-    wave_lds_sync();
-#pragma unroll
-    for (int k = 0; k < kChunks; ++k) {
-      const int j = 64 * k + lane;
-      ln[k] = 0;
-      if (j < num_old) {
-        const I lep = leps.get(j);
-        backward_ext_ks(x, lep, base, ex[k]);
-        ex[k].m = m - 1;
-        ex[k].n = lep.n;
-        ln[k] = lep.n - lep.m + 1;
-      }
-    }
-    P curr = min_seed_intv;
-    bool collected = false;
-    int nl = 0;
-    uint64_t keep[kChunks];
-#pragma unroll
-    for (int k = 0; k < kChunks; ++k) {
-      keep[k] = 0;
-      const int n = num_old - 64 * k < 64 ? num_old - 64 * k : 64;
-      for (int b = 0; b < n; ++b) {
-        const P sb = lane_read(ex[k].s, b);
-        if (sb >= curr) {
-          keep[k] |= 1ull << b;
-          ++nl;
-          curr = sb;
-        } else if (!collected && lane_read(ln[k], b) >= o.min_seed_len) {
-          if (ns == cap_s) return -1;
-          seeds.put(ns++, leps.get(64 * k + b));  // every lane stores the same entry
-          collected = true;
-        }
-      }
-    }
-    wave_lds_sync();  // every entry was read above
-    int before = 0;
-#pragma unroll
-    for (int k = 0; k < kChunks; ++k) {
-      if ((keep[k] >> lane) & 1) leps.put(before + __popcll(keep[k] & ((1ull << lane) - 1)), ex[k]);
-      before += __popcll(keep[k]);
-    }
-    wave_lds_sync();
-    return nl;
-  }
-};
-
-// Slow path for the reads listed in `list`, one wavefront per read: LEP
-// lists of kSlowLep entries in LDS, which no read of <= 320 bases can
-// outgrow, the backward steps on the wavefront's lanes (WaveBack) and the
-// rest of the search on every lane alike.  Pass 0 counts and keeps the first
-// 2 * kSlowLep intervals in the read's scratch; pass 1 puts all intervals at
-// the pool offsets computed from the counts, copying them from the scratch
-// when it still holds them all (`from_scratch`: every slow read had its own
-// scratch in pass 0) and searching again otherwise.
-__global__ void __launch_bounds__(64) k_seed_slow(SeedArgs a, const int32_t *list, int n_list, const int32_t *n_dev,
-                                                  int c0, Intv *scratch, const int64_t *pool_off, Intv *pool, int pass,
-                                                  int from_scratch) {
-  if (a.stop && *a.stop) return;  // a capacity check before this kernel failed: the batch is redone
-  __shared__ LepWide lds_a[kSlowLep], lds_f[kSlowLep];
-  const int t = blockIdx.x, lane = threadIdx.x;
-  int nv = n_list;
-  if (n_dev) {
-    const int m = *n_dev - c0;
-    nv = m < 0 ? 0 : m < n_list ? m : n_list;
-  }
-  if (t >= nv) return;  // the whole wavefront
-  const int r = list[t];
-  const int off = a.off[r], len = a.off[r + 1] - off;
-  const uint8_t *q = a.seq + off;
-  Intv *sc = scratch + (int64_t)t * kSlowScratch;
-  if (pass && from_scratch && a.n_intv[r] <= 2 * kSlowLep) {
-    const Intv *src = sc + 3 * kSlowLep;
-    Intv *dst = pool + pool_off[t];
-    for (int k = lane, n = a.n_intv[r]; k < n; k += 64) dst[k] = src[k];
-    return;
-  }
-  Intv *slot = pass ? pool + pool_off[t] : sc + 3 * kSlowLep;
-  const int cap = pass ? (int)(pool_off[t + 1] - pool_off[t]) : 2 * kSlowLep;
-  IntvSink sink{slot, cap, 0, 0, a.opt.max_occ};  // every lane pushes the same intervals
-  GlobalBuf<LepWide> buf{GlobalList<LepWide>{lds_a}, GlobalList<LepWide>{lds_f}, kSlowLep, kSlowLep};
-  if (!smem_round1<true, GlobalBuf<LepWide>, WaveBack>(a.idx, a.opt, q, len, sink, buf, nullptr)) {
-    sink.n = 0;
-    sink.n_seed = 0;
-    smem_round1_per_end(a.idx, a.opt, q, len, sink, nullptr);
-  }
-  const int nsm = sink.n;
-  for (int k = 0; k < nsm; ++k) {
-    const Intv smem = slot[k];
-    reseed_one<GlobalList<LepWide>, GlobalList<LepWide>, WaveBack>(a.idx, a.opt, q, len, smem, buf.a, buf.f,
-                                                                    kSlowLep, kSlowLep, sink, nullptr);
-  }
-  reseed_round3<int64_t>(a.idx, a.opt, q, len, sink, nullptr);
-  if (lane == 0) {
-    a.n_intv[r] = sink.n;
-    a.n_seed[r] = sink.n_seed;
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1561,17 +1265,20 @@ __global__ void __launch_bounds__(256) k_ext_finish(ExtFinishArgs a) {
 }
 
 // k-mer table: thread per k-mer code
-__global__ void __launch_bounds__(256) k_kmer_table(DevIndex x, uint32_t *table) {
+template <class T>
+__global__ void __launch_bounds__(256) k_kmer_table(DevIndex x, T *table) {
   const uint32_t code = blockIdx.x * blockDim.x + threadIdx.x;
-  if (code >= (1u << (2 * kKmer))) return;
-  uint32_t e[3];
+  if (code >> (2 * kKmer)) return;
+  T e[3];
   kmer_interval(x, code, e);
-  table[3 * (size_t)code] = e[0];
-  table[3 * (size_t)code + 1] = e[1];
-  table[3 * (size_t)code + 2] = e[2];
+  T *o = table + 3 * (uint64_t)code;
+  for (int i = 0; i < 3; ++i) o[i] = e[i];
 }
 void launch_kmer_table(const DevIndex &x, uint32_t *table, hipStream_t s) {
-  hipLaunchKernelGGL(k_kmer_table, dim3((1u << (2 * kKmer)) / 256), dim3(256), 0, s, x, table);
+  hipLaunchKernelGGL(k_kmer_table<uint32_t>, dim3((1u << (2 * kKmer)) / 256), dim3(256), 0, s, x, table);
+}
+void launch_kmer_table64(const DevIndex &x, int64_t *table, hipStream_t s) {
+  hipLaunchKernelGGL(k_kmer_table<int64_t>, dim3((1u << (2 * kKmer)) / 256), dim3(256), 0, s, x, table);
 }
 
 // Occ lines built on the device from the BWA .bwt body: thread per line
@@ -1868,72 +1575,6 @@ __global__ void __launch_bounds__(64) k_traceback(TbArgs a) {
 // ---------------------------------------------------------------------------
 static inline unsigned blocks(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
-// 16-byte list entries when every SA row fits 32 bits
-// the narrow layout is in use (texts below 2^32 rows, unless the context
-// was set to the wide layout): decided by the index, not by the text size
-static bool seed_narrow(const DevIndex &x) { return x.occn != nullptr && x.sbc != nullptr; }
-static size_t seed_lds_bytes(const DevIndex &x) {
-  return seed_narrow(x) ? (size_t)((((uint64_t)x.n + 1) >> 21) + 1) * 16 : 0;
-}
-int seed_grid_threads(int n_cu, const DevIndex &x, int block) {
-  int per_cu = 0;
-  hipError_t e = seed_narrow(x)
-                     ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_seed<LepNarrow, false>, block,
-                                                                    seed_lds_bytes(x))
-                     : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_seed<LepWide, false>, block, 0);
-  if (e != hipSuccess || per_cu < 1) per_cu = 1024 / block;
-  return n_cu * per_cu * block;
-}
-void launch_seed(const SeedArgs &a, int n_threads, int blocks_per_cu, int block, hipStream_t s) {
-  if (!a.n_reads) return;
-  const int need = blocks(a.n_reads, block), have = n_threads / block;
-  int nb = need < have ? need : have;
-  if (nb < 1) nb = 1;
-  if (seed_narrow(a.idx)) {
-    void (*kern)(SeedArgs) = a.idx.saf ? k_seed<LepNarrow, true> : k_seed<LepNarrow, false>;
-    // The compute unit's LDS (160 KB) is shared by the blocks it is to hold,
-    // and each block keeps one copy of the superblock counts, so larger
-    // blocks leave more room for list entries; the LEP entries per thread are
-    // the most that still lets that many blocks be resident (a block that is
-    // not resident would only start when another finishes, doubling the
-    // kernel's time).
-    const size_t sb = seed_lds_bytes(a.idx);
-    int dev = 0, n_cu = 0, max_lds = 65536;
-    if (hipGetDevice(&dev) == hipSuccess) {
-      hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev);
-      if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
-          max_lds < 16384)
-        max_lds = 65536;
-    }
-    int want = blocks_per_cu;
-    if (want <= 0 && (hipOccupancyMaxActiveBlocksPerMultiprocessor(&want, kern, block, sb) != hipSuccess || want < 1))
-      want = 1024 / block;
-    size_t per_block = (size_t)160 * 1024 / (size_t)want - 1024;  // slack for allocation granules
-    per_block = per_block < (size_t)max_lds ? per_block : (size_t)max_lds;
-    int capl = per_block > sb ? (int)((per_block - sb) / ((size_t)block * 12)) : 0;
-    capl = capl < kLepCap ? capl : kLepCap;
-    int resident = 0;
-    for (; capl > 0; --capl) {
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kern, block, sb + (size_t)capl * block * 12) !=
-          hipSuccess)
-        resident = 0;
-      if (resident >= want) break;
-    }
-    // no more blocks than the compute units hold at once
-    if (n_cu > 0 && resident > 0 && nb > resident * n_cu) nb = resident * n_cu;
-    SeedArgs b = a;
-    b.lep_lds = capl;
-    hipLaunchKernelGGL(kern, dim3(nb), dim3(block), sb + (size_t)capl * block * 12, s, b);
-  } else {
-    hipLaunchKernelGGL((k_seed<LepWide, false>), dim3(nb), dim3(block), 0, s, a);
-  }
-}
-void launch_seed_slow(const SeedArgs &a, const int32_t *list, int n_list, const int32_t *n_dev, int c0, Intv *scratch,
-                      const int64_t *pool_off, Intv *pool, int pass, int from_scratch, hipStream_t s) {
-  if (n_list)
-    hipLaunchKernelGGL(k_seed_slow, dim3(n_list), dim3(64), 0, s, a, list, n_list, n_dev, c0, scratch, pool_off, pool,
-                       pass, from_scratch);
-}
 void launch_sa_lookup(const SaArgs &a, hipStream_t s) {
   if (a.total) hipLaunchKernelGGL(k_sa_lookup, dim3(blocks(a.total, 256)), dim3(256), 0, s, a);
 }

@@ -240,8 +240,8 @@ int g3a_set_tuning(g3a_ctx *ctx, int strip_rows, int lane_blocks_per_cu, int wav
  * reference counterpart. */
 int g3a_set_ext_packed(g3a_ctx *ctx, int packed);
 /* Index layout of texts of 2^32 rows or more (32-byte Occ lines of 64 rows
- * with 2^32-row superblocks, 64-bit intervals in seeding, no 12-mer table,
- * no learned form), used on any text when on = 1; called before
+ * with 2^32-row superblocks, 64-bit intervals in seeding and in the 12-mer
+ * table, no learned form), used on any text when on = 1; called before
  * g3a_memcpy_index.  Output is identical.  For tests of that layout on texts
  * small enough to check.  No reference counterpart. */
 int g3a_set_wide_layout(g3a_ctx *ctx, int on);
@@ -255,16 +255,13 @@ int g3a_ext_packed(const g3a_ctx *ctx);
  * counterpart. */
 int g3a_autotune(g3a_ctx *ctx, int *strip_rows, int *lane_blocks_per_cu, float *best_ms);
 /* Persistent seeding blocks per compute unit at the current block size
- * (g3a_set_seed_grid); 0: the occupancy maximum.  Each block's share of the
- * compute unit's LDS holds the first entries of its threads' LEP lists (the
- * rest spill to a global slice per thread), so the grid trades latency
- * hiding against list traffic.  No reference counterpart. */
+ * (g3a_set_seed_grid); 0: the occupancy maximum.  No reference counterpart. */
 int g3a_set_seed_blocks(g3a_ctx *ctx, int blocks_per_cu);
 /* The seeding grid in full: threads per block (a multiple of 64, at most
  * 1024; default 1024) and blocks per compute unit (0: the occupancy maximum;
- * default 1).  Each block keeps one
- * copy of the Occ superblock counts in LDS, so larger blocks leave more of
- * the compute unit's LDS to the threads' lists.  No reference counterpart. */
+ * default 1).  16 threads work on a read, and each block keeps one copy of
+ * the Occ superblock counts in LDS; a batch that would leave compute units
+ * without a block runs in smaller ones.  No reference counterpart. */
 int g3a_set_seed_grid(g3a_ctx *ctx, int threads_per_block, int blocks_per_cu);
 /* Seeding order: 1 seeds the reads in the order of a minimizer
  * key (the smallest hash over each read's canonical 16-mers), so that
@@ -279,9 +276,7 @@ int g3a_set_seed_order(g3a_ctx *ctx, int ordered);
 int g3a_set_chain_serial(g3a_ctx *ctx, int on);
 /* Seeding autotuner: re-aligns the batch last aligned once per seeding grid
  * (threads per block x blocks per compute unit: 1024x1, 512x2, 256x4, 128x6;
- * each block keeps one copy of the superblock counts in LDS and the rest of
- * its share holds the first entries of its threads' LEP lists, so fewer,
- * larger blocks keep more in LDS) and order (input, minimizer), keeps the
+ * each block keeps one copy of the superblock counts in LDS) and order (input, minimizer), keeps the
  * setting with the fastest seeding stage and reports it with its time.  The
  * batch's output is identical for every setting.  No reference counterpart. */
 int g3a_autotune_seed(g3a_ctx *ctx, int *threads_per_block, int *blocks_per_cu, int *ordered, float *best_ms);
