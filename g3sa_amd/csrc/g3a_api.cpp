@@ -48,7 +48,7 @@ struct DevBuf {
 // on a second one whose buffers are views into the device's static scratch
 // array.
 struct Work {
-  DevBuf eh_pool, tb_order, tb_ctr, tb_nw;
+  DevBuf eh_pool, tb_order, tb_ctr;
   DevBuf seed_key, seed_key2, seed_idx, seed_order, seed_sort_tmp;  // seeding order
   // seeding
   DevBuf intv, n_intv, n_seed, slow, intv_base, seed_off, counters, slow_list, slow_scratch, slow_n, slow_off;
@@ -544,7 +544,6 @@ static int alloc_alns(g3a_ctx *ctx, int64_t T_a) {
          ensure(ctx, ctx->w->cig_size, (size_t)T_a * 8) || ensure(ctx, ctx->w->z_off, (size_t)(T_a + 1) * 8) ||
          ensure(ctx, ctx->w->cig_off, (size_t)(T_a + 1) * 8) || ensure(ctx, ctx->w->alns, (size_t)T_a * sizeof(Aln)) ||
          ensure(ctx, ctx->w->scan_tmp, scan_tmp_bytes(T_a + 1)) || ensure(ctx, ctx->w->tb_order, (size_t)T_a * 4 + 4) ||
-         ensure(ctx, ctx->w->tb_nw, (size_t)T_a * 4 + 4) ||
          ensure(ctx, ctx->w->tb_ctr, 64) || ensure(ctx, ctx->w->eh_pool, (size_t)traceback_pool_words(ctx->run_tb_threads) * 4);
 }
 
@@ -1054,7 +1053,6 @@ static int enqueue_batch(g3a_ctx *ctx, int n, const Caps &c, bool timed) {
   tb.eh_pool = P<int32_t>(w.eh_pool);
   tb.tb_order = P<int32_t>(w.tb_order);
   tb.tb_ctr = P<int32_t>(w.tb_ctr);
-  tb.tb_nw = P<int32_t>(w.tb_nw);
   if (timed) HIPCK(hipEventRecord(ctx->kev[10], s));
   launch_traceback(tb, ctx->run_tb_threads, ctx->n_cu, s);
   if (timed) HIPCK(hipEventRecord(ctx->kev[11], s));
@@ -1851,7 +1849,7 @@ void g3a_destroy(g3a_ctx *ctx) {
                     &ctx->own.seed_order, &ctx->own.seed_sort_tmp,
                     &ctx->own.ext_res[0], &ctx->own.ext_res[1], &ctx->own.ext_key, &ctx->own.ext_hist, &ctx->own.totals,
                     &ctx->own.ext_sorted, &ctx->own.ext_slow, &ctx->own.ext_ctr, &ctx->own.ext_rowbuf,
-                    &ctx->own.eh_pool, &ctx->own.tb_order, &ctx->own.tb_ctr, &ctx->own.tb_nw, &ctx->li_saf, &ctx->li_keys,
+                    &ctx->own.eh_pool, &ctx->own.tb_order, &ctx->own.tb_ctr, &ctx->li_saf, &ctx->li_keys,
                     &ctx->li_root, &ctx->li_leaf, &ctx->li_knot, &ctx->li_leaf_a, &ctx->li_short, &ctx->li_ctr,
                     &ctx->ctg_names, &ctx->ctg_name_off, &ctx->log_tab, &ctx->names, &ctx->name_off, &ctx->quals,
                     &ctx->qual_off, &ctx->txt_len, &ctx->txt_off, &ctx->txt, &ctx->txt_bound, &ctx->stage_off, &ctx->txt_stage, &ctx->fmt_flag, &ctx->mapq, &ctx->md_len,

@@ -1832,28 +1832,11 @@ G3A_HD int push_cigar(uint32_t *cigar, int n, int op, int len) {
 // used.  `tq`/`tt` give query/target bases; eh_h/eh_e hold qlen+1 entries and
 // z holds tlen*min(qlen, 2w+1) direction bytes.  Returns the score.
 // Row buffers of the banded global alignment: H and E of the previous row
-// by query column.  EhArray keeps whole rows; EhRing keeps a ring of RB
-// columns (enough when 2w+2 <= RB) at a stride, e.g. one lane's slice of a
-// wavefront's LDS block.
+// by query column.
 struct EhArray {
-  static constexpr bool kStage = false;
   int32_t *h, *e;
   G3A_HD int32_t &H(int j) { return h[j]; }
   G3A_HD int32_t &E(int j) { return e[j]; }
-};
-// The ring also carries `zst`, RB bytes (16-byte aligned) where a row's
-// direction bytes are gathered before they are stored 16 bytes at a time:
-// a thread's row is then whole 16-byte pieces of its alignment's matrix
-// instead of 4-byte pieces, which the memory side merges far better when
-// every lane of a wavefront writes its own alignment.
-template <int RB>
-struct EhRing {
-  static constexpr bool kStage = true;
-  int32_t *h, *e;
-  int stride;
-  uint32_t *zst;
-  G3A_HD int32_t &H(int j) { return h[(j & (RB - 1)) * stride]; }
-  G3A_HD int32_t &E(int j) { return e[(j & (RB - 1)) * stride]; }
 };
 
 // z-matrix row stride: the band's column count rounded up to 16 bytes
@@ -1863,9 +1846,8 @@ G3A_HD int z_stride(int qlen, int w) {
 }
 
 // ksw_global2 (bwa/src/ksw.cu:706-812, DR-9): banded global alignment.
-// global_dp fills the direction bytes (a row's written four at a time, or
-// gathered in eh.zst and written sixteen at a time) and returns the score;
-// global_walk turns them into the CIGAR.
+// global_dp fills the direction bytes (a row's written four at a time) and
+// returns the score; global_walk turns them into the CIGAR.
 template <class Q, class T, class EH>
 G3A_HD int global_dp(const Opt &o, int qlen, Q tq, int tlen, T tt, int w, EH eh, uint8_t *z) {
   const int MINUS_INF = -0x40000000;
@@ -1906,24 +1888,11 @@ G3A_HD int global_dp(const Opt &o, int qlen, Q tq, int tlen, T tt, int w, EH eh,
       const int c = j - beg;
       zw |= d << (8 * (c & 3));
       if ((c & 3) == 3) {
-        if constexpr (EH::kStage) eh.zst[c >> 2] = zw;
-        else zi[c >> 2] = zw;
+        zi[c >> 2] = zw;
         zw = 0;
       }
     }
-    if constexpr (EH::kStage) {
-      if ((end - beg) & 3) eh.zst[(end - beg) >> 2] = zw;
-      // the row's words, whole 16-byte pieces (bytes past the band are
-      // never read)
-#if defined(__HIPCC__)
-      for (int q = 0; q < ((end - beg + 15) >> 4); ++q)
-        reinterpret_cast<uint4 *>(zi)[q] = reinterpret_cast<const uint4 *>(eh.zst)[q];
-#else
-      for (int q = 0; q < ((end - beg + 15) >> 4) * 4; ++q) zi[q] = eh.zst[q];
-#endif
-    } else {
-      if ((end - beg) & 3) zi[(end - beg) >> 2] = zw;
-    }
+    if ((end - beg) & 3) zi[(end - beg) >> 2] = zw;
     eh.H(end) = h1;
     eh.E(end) = MINUS_INF;
   }
@@ -1971,12 +1940,12 @@ G3A_HD int64_t aln_z_size(int lq, int64_t rlen, int w) {
 // kept region of a read of length l_seq.  `read` is the read, `cig` has
 // aln_cigar_cap() words (the core CIGAR at aln_core_at()), z has
 // aln_z_size() bytes, eh_h/eh_e lq+1 entries.
-// pre_nw: when not null, the direction bytes and the score (*pre_nw) of the
-// global alignment are already computed (k_tb_wave_dp) and only the walk runs.
+// pre: when not null, the global alignment is done (g3a_trace.h): its
+// n_core, nw_score and nm are in *pre and the core CIGAR is in place.
 template <class EH>
 G3A_HD void trace_and_finalize(const DevIndex &x, const Opt &o, const uint8_t *read, int l_seq, const Region &g,
                                int ai, EH eh, uint8_t *z, uint32_t *cig, int64_t cig_base, Aln &a,
-                               const int32_t *pre_nw = nullptr) {
+                               const Aln *pre = nullptr) {
   const int64_t l_pac = x.l_pac;
   const int lq = g.qe - g.qb;
   const int64_t rlen = g.re - g.rb;
@@ -1989,7 +1958,11 @@ G3A_HD void trace_and_finalize(const DevIndex &x, const Opt &o, const uint8_t *r
   TextReader tr(x.pac, l_pac);
   // NM as the reference's traceback counts it (aux.cu:2910-2941)
   int n_mm = 0, n_gap = 0;
-  if (w == 0) {
+  if (pre) {
+    n_core = pre->n_core;
+    nw = pre->nw_score;
+    n_mm = pre->nm;
+  } else if (w == 0) {
     // one ungapped pass: score and mismatches together
     core[0] = (uint32_t)(lq << 4);
     n_core = 1;
@@ -2001,9 +1974,8 @@ G3A_HD void trace_and_finalize(const DevIndex &x, const Opt &o, const uint8_t *r
     }
   } else {
     // the band revisits each query byte on 2w+1 rows: plain loads (cached)
-    nw = pre_nw ? *pre_nw
-                : global_dp(o, lq, [&](int j) { return (int)query[j]; }, (int)rlen, [&](int i) { return tr(rb + i); },
-                            w, eh, z);
+    nw = global_dp(o, lq, [&](int j) { return (int)query[j]; }, (int)rlen, [&](int i) { return tr(rb + i); }, w, eh,
+                   z);
     n_core = global_walk(lq, (int)rlen, w, z, core);
     TextReader trn(x.pac, l_pac);
     ByteReader qn(query);

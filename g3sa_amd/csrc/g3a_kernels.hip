@@ -1,5 +1,5 @@
 // HIP kernels of the BWA-MEM hot path for MI355X (gfx950, wave64); seeding is
-// in g3a_seed.hip.
+// in g3a_seed.hip, the traceback in g3a_trace.hip.
 //
 // Stage kernels (one launch each, all on the context's stream):
 //   k_sa_lookup      thread per seed: SA interval row -> reference position
@@ -10,7 +10,6 @@
 //                    then right, anti-diagonal sweep over 64-row tiles
 //   k_region_filter  thread per read
 //   k_aln_prep       thread per read: kept regions -> alignment list
-//   k_traceback      thread per alignment: global alignment + finalize
 #include "g3a_dev.h"
 #include "g3a_kernels.h"
 
@@ -1344,232 +1343,6 @@ __global__ void __launch_bounds__(128) k_aln_prep(AlnPrepArgs a) {
   }
 }
 
-// Alignment order for k_traceback: those that need the banded global
-// alignment (w > 0) first, the ungapped ones (w = 0) last, so that the DP
-// loops of a wavefront run with all lanes busy.
-// Traceback classes by band: 0: 2w+2 <= 16, 1: <= 32, 2: wider (w > 0),
-// 3: ungapped (w = 0).  The row buffers of class c < 2 fit an LDS ring of
-// 16 << c columns per lane, so the smaller classes run at higher occupancy.
-__device__ __forceinline__ int tb_class(const TbArgs &a, int64_t t) {
-  const Region g = a.aln_reg[t];
-  const int w = global_bw(a.opt, g.qe - g.qb, g.re - g.rb, g.score);
-  return w == 0 ? 3 : 2 * w + 2 <= 16 ? 0 : 2 * w + 2 <= 32 ? 1 : 2;
-}
-// tb_ctr[0..2]: alignments of classes 0..2 (tiles of kTilePer * 256)
-__global__ void __launch_bounds__(256) k_tb_count(TbArgs a) {
-  if (a.stop && *a.stop) return;  // a capacity check before this kernel failed: the batch is redone
-  __shared__ int32_t cnt[3];
-  if (threadIdx.x < 3) cnt[threadIdx.x] = 0;
-  __syncthreads();
-  const int64_t tile = (int64_t)blockIdx.x * (256 * kTilePer);
-  const int64_t n = dcount(a.n_dev, a.n_alns);
-  int c3[3] = {0, 0, 0};
-#pragma unroll
-  for (int i = 0; i < kTilePer; ++i) {
-    const int64_t t = tile + i * 256 + threadIdx.x;
-    const int c = t < n ? tb_class(a, t) : 3;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) c3[k] += c == k;
-  }
-#pragma unroll
-  for (int k = 0; k < 3; ++k)
-    if (c3[k]) atomicAdd(&cnt[k], c3[k]);
-  __syncthreads();
-  if (threadIdx.x < 3 && cnt[threadIdx.x]) atomicAdd(a.tb_ctr + threadIdx.x, cnt[threadIdx.x]);
-}
-// The list holds classes 0, 1, 2 in turn from the front and class 3 from the
-// back; tb_ctr[4..7] are the placement cursors (tiles of kTilePer * 256).
-__global__ void __launch_bounds__(256) k_tb_order(TbArgs a) {
-  if (a.stop && *a.stop) return;  // a capacity check before this kernel failed: the batch is redone
-  __shared__ int32_t cnt[4], base[4];
-  if (threadIdx.x < 4) cnt[threadIdx.x] = 0;
-  __syncthreads();
-  const int64_t tile = (int64_t)blockIdx.x * (256 * kTilePer);
-  const int64_t n_alns = dcount(a.n_dev, a.n_alns);
-  int cls[kTilePer], at[kTilePer];
-#pragma unroll
-  for (int i = 0; i < kTilePer; ++i) {
-    const int64_t t = tile + i * 256 + threadIdx.x;
-    cls[i] = t < n_alns ? tb_class(a, t) : -1;
-    at[i] = cls[i] >= 0 ? atomicAdd(&cnt[cls[i]], 1) : -1;
-  }
-  __syncthreads();
-  if (threadIdx.x < 4) base[threadIdx.x] = cnt[threadIdx.x] ? atomicAdd(a.tb_ctr + 4 + threadIdx.x, cnt[threadIdx.x]) : 0;
-  __syncthreads();
-  const int64_t base1 = a.tb_ctr[0], base2 = base1 + a.tb_ctr[1];
-#pragma unroll
-  for (int i = 0; i < kTilePer; ++i) {
-    const int c = cls[i];
-    if (c < 0) continue;
-    const int r = base[c] + at[i];
-    const int64_t pos = c == 0 ? r : c == 1 ? base1 + r : c == 2 ? base2 + r : n_alns - 1 - r;
-    a.tb_order[pos] = (int32_t)(tile + i * 256 + threadIdx.x);
-  }
-}
-
-// Persistent grids over the ordered list.  k_traceback_dp<RB> takes one
-// class: its row buffers are an RB-column ring per lane in LDS (lanes
-// interleaved), or for the widest class with 2w+2 > RB the thread's slice of
-// the global pool (2 * kQMax words, contiguous per thread); k_traceback takes
-// the ungapped class.
-template <int RB>
-__global__ void __launch_bounds__(64) k_traceback_dp(TbArgs a, int cls) {
-  if (a.stop && *a.stop) return;  // a capacity check before this kernel failed: the batch is redone
-  __shared__ int32_t ring_h[RB * 64], ring_e[RB * 64];
-  __shared__ uint4 zstage[64 * RB / 16];  // each lane's row of direction bytes, RB bytes
-  const int lane = threadIdx.x;
-  const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + lane;
-  const int64_t nthreads = (int64_t)gridDim.x * blockDim.x;
-  int32_t *eh_h = a.eh_pool + gtid * 2 * kQMax, *eh_e = eh_h + kQMax;
-  int64_t e0 = 0;
-  for (int k = 0; k < cls; ++k) e0 += a.tb_ctr[k];
-  const int64_t e1 = e0 + a.tb_ctr[cls];
-  for (int64_t e = e0 + gtid; e < e1; e += nthreads) {
-    const int64_t t = a.tb_order[e];
-    const int r = a.aln_read[t];
-    const int off = a.off[r], l_seq = a.off[r + 1] - off;
-    const Region g = a.aln_reg[t];
-    const int w = global_bw(a.opt, g.qe - g.qb, g.re - g.rb, g.score);
-    Aln out;
-    if (RB == 64 && 2 * w + 1 <= 128)  // direction bytes and score from k_tb_wave_dp
-      trace_and_finalize(a.idx, a.opt, a.seq + off, l_seq, g, a.aln_rank[t], EhArray{eh_h, eh_e},
-                         a.z + a.z_off[t], a.cigar + a.cig_off[t], a.cig_off[t], out, a.tb_nw + t);
-    else if (2 * w + 2 <= RB)
-      trace_and_finalize(a.idx, a.opt, a.seq + off, l_seq, g, a.aln_rank[t],
-                         EhRing<RB>{ring_h + lane, ring_e + lane, 64,
-                                    reinterpret_cast<uint32_t *>(zstage + lane * (RB / 16))},
-                         a.z + a.z_off[t], a.cigar + a.cig_off[t], a.cig_off[t], out);
-    else
-      trace_and_finalize(a.idx, a.opt, a.seq + off, l_seq, g, a.aln_rank[t], EhArray{eh_h, eh_e},
-                         a.z + a.z_off[t], a.cigar + a.cig_off[t], a.cig_off[t], out);
-    a.alns[t] = out;
-  }
-}
-
-// Banded global DP (global_dp's recurrence, ksw_global2, DR-9) of the
-// widest class's alignments with 64 (NH - 1) < 2w+1 <= 64 NH band columns:
-// one wavefront per alignment, lane L on columns beg + L + 64 h (h < NH) of
-// each row.  F depends only on the row's M values, so a row is one max-plus
-// prefix scan over the columns (F_c = max(-inf - c e, max_{c' < c} M_c' - o
-// - e (c - c'))), carried from one 64-column half to the next; E and the
-// next row's H come from neighbouring columns, shifted by the band's start.
-// Writes the direction bytes and the score (tb_nw) that k_traceback_dp<64>
-// then walks; identical to global_dp on every cell.
-template <int NH>
-__device__ __forceinline__ int col_get(const int (&v)[NH], int c) {
-  int r = __shfl(v[0], c & 63);
-  if (NH > 1) {
-    const int r1 = __shfl(v[NH - 1], c & 63);
-    r = c >= 64 ? r1 : r;
-  }
-  return r;
-}
-template <int NH>
-__global__ void __launch_bounds__(256) k_tb_wave_dp(TbArgs a) {
-  if (a.stop && *a.stop) return;  // a capacity check before this kernel failed: the batch is redone
-  const int L = threadIdx.x & 63;
-  const int64_t wid = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) >> 6;
-  const int64_t e0 = (int64_t)a.tb_ctr[0] + a.tb_ctr[1], e1 = e0 + a.tb_ctr[2];
-  const Opt &o = a.opt;
-  const int MINUS_INF = -0x40000000;
-  const int oe_del = o.o_del + o.e_del, oe_ins = o.o_ins + o.e_ins;
-  for (int64_t e = e0 + wid; e < e1; e += nwaves) {
-    const int64_t t = a.tb_order[e];
-    const Region g = a.aln_reg[t];
-    const int qlen = g.qe - g.qb, tlen = (int)(g.re - g.rb);
-    const int w = global_bw(o, qlen, tlen, g.score);
-    if (2 * w + 1 > 64 * NH || 2 * w + 1 <= 64 * (NH - 1)) continue;  // another launch's alignment
-    const int r = a.aln_read[t];
-    const uint8_t *query = a.seq + a.off[r] + g.qb;
-    uint8_t *z = a.z + a.z_off[t];
-    const int zs = z_stride(qlen, w);
-    TextReader tr(a.idx.pac, a.idx.l_pac);
-    int hp[NH], ep[NH], beg_p = 0, n_p = 0;
-#pragma unroll
-    for (int h = 0; h < NH; ++h) {
-      hp[h] = 0;
-      ep[h] = MINUS_INF;
-    }
-    for (int i = 0; i < tlen; ++i) {
-      const int beg = i > w ? i - w : 0, end = i + w + 1 < qlen ? i + w + 1 : qlen, n = end - beg;
-      const ScoreRow sr = score_row(o, tr(g.rb + i));
-      int m[NH], pm[NH], ein[NH];
-#pragma unroll
-      for (int h = 0; h < NH; ++h) {
-        const int c = 64 * h + L, j = beg + c;
-        const bool act = c < n;
-        const int qj = act ? (int)query[j] : 4;
-        int hd;
-        if (i == 0) {
-          hd = j == 0 ? 0 : -(o.o_ins + o.e_ins * j);
-          ein[h] = MINUS_INF;
-        } else {
-          const int delta = beg - beg_p, kp = c - 1 + delta, ke = c + delta;
-          const int hs = col_get<NH>(hp, kp < 0 ? 0 : kp), es = col_get<NH>(ep, ke > 64 * NH - 1 ? 64 * NH - 1 : ke);
-          hd = kp < 0 ? (beg_p == 0 ? -(o.o_del + o.e_del * i) : MINUS_INF) : hs;
-          ein[h] = ke >= n_p ? MINUS_INF : es;
-        }
-        m[h] = hd + sr(qj);
-        pm[h] = act ? m[h] - oe_ins + o.e_ins * (c + 1) : MINUS_INF;
-      }
-      // inclusive max scan of each half, the second carried by the first's total
-#pragma unroll
-      for (int h = 0; h < NH; ++h) {
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-          const int u = __shfl_up(pm[h], d);
-          pm[h] = L >= d && u > pm[h] ? u : pm[h];
-        }
-      }
-      int carry = MINUS_INF;
-#pragma unroll
-      for (int h = 0; h < NH; ++h) {
-        pm[h] = carry > pm[h] ? carry : pm[h];
-        int ex = __shfl_up(pm[h], 1);
-        ex = L == 0 ? carry : ex;
-        ex = ex < MINUS_INF ? MINUS_INF : ex;
-        carry = __shfl(pm[h], 63);
-        const int c = 64 * h + L;
-        const int f = ex - c * o.e_ins;
-        int dir = m[h] >= ein[h] ? 0 : 1, hh = m[h] >= ein[h] ? m[h] : ein[h];
-        dir = hh >= f ? dir : 2;
-        hh = hh >= f ? hh : f;
-        int tt = m[h] - oe_del, e2 = ein[h] - o.e_del;
-        dir |= e2 > tt ? 4 : 0;
-        e2 = e2 > tt ? e2 : tt;
-        tt = m[h] - oe_ins;
-        dir |= f - o.e_ins > tt ? 32 : 0;
-        if (c < n) z[(int64_t)i * zs + c] = (uint8_t)dir;
-        hp[h] = hh;
-        ep[h] = e2;
-      }
-      beg_p = beg;
-      n_p = n;
-    }
-    const int score = col_get<NH>(hp, qlen - 1 - beg_p);
-    if (L == 0) a.tb_nw[t] = score;
-  }
-}
-
-__global__ void __launch_bounds__(64) k_traceback(TbArgs a) {
-  if (a.stop && *a.stop) return;  // a capacity check before this kernel failed: the batch is redone
-  const int64_t gtid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t nthreads = (int64_t)gridDim.x * blockDim.x;
-  int32_t *eh_h = a.eh_pool + gtid * 2 * kQMax, *eh_e = eh_h + kQMax;
-  const int64_t n_alns = dcount(a.n_dev, a.n_alns);
-  for (int64_t e = a.tb_ctr[0] + a.tb_ctr[1] + a.tb_ctr[2] + gtid; e < n_alns; e += nthreads) {
-    const int64_t t = a.tb_order[e];
-    const int r = a.aln_read[t];
-    const int off = a.off[r], l_seq = a.off[r + 1] - off;
-    const Region g = a.aln_reg[t];
-    Aln out;
-    trace_and_finalize(a.idx, a.opt, a.seq + off, l_seq, g, a.aln_rank[t], EhArray{eh_h, eh_e}, a.z + a.z_off[t],
-                       a.cigar + a.cig_off[t], a.cig_off[t], out);
-    a.alns[t] = out;
-  }
-}
-
 // ---------------------------------------------------------------------------
 // launch helpers
 // ---------------------------------------------------------------------------
@@ -1625,40 +1398,6 @@ void launch_region_filter(const RegionArgs &a, hipStream_t s) {
 void launch_aln_prep(const AlnPrepArgs &a, hipStream_t s) {
   if (a.n_reads) hipLaunchKernelGGL(k_aln_prep, dim3(blocks(a.n_reads, 128)), dim3(128), 0, s, a);
 }
-int traceback_grid_threads(int n_cu) {
-  int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_traceback, 64, 0) != hipSuccess || per_cu < 1)
-    per_cu = 16;
-  return n_cu * per_cu * 64;
-}
-int64_t traceback_pool_words(int n_threads) { return (int64_t)n_threads * 2 * kQMax; }
-void launch_traceback(const TbArgs &a, int n_threads, int n_cu, hipStream_t s) {
-  if (!a.n_alns) return;
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, s, a.tb_ctr, 8, 0);
-  const dim3 gt((unsigned)((a.n_alns + 256 * kTilePer - 1) / (256 * kTilePer)));
-  hipLaunchKernelGGL(k_tb_count, gt, dim3(256), 0, s, a);
-  hipLaunchKernelGGL(k_tb_order, gt, dim3(256), 0, s, a);
-  // the pool has a slice for each of the n_threads threads
-  auto dp_blocks = [&](const void *k) {
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, 64, 0) != hipSuccess || per_cu < 1) per_cu = 4;
-    int b = n_cu * per_cu;
-    if (b > n_threads / 64) b = n_threads / 64;
-    return b < 1 ? 1 : b;
-  };
-  hipLaunchKernelGGL(k_traceback_dp<16>, dim3((unsigned)dp_blocks((const void *)k_traceback_dp<16>)), dim3(64), 0, s,
-                     a, 0);
-  hipLaunchKernelGGL(k_traceback_dp<32>, dim3((unsigned)dp_blocks((const void *)k_traceback_dp<32>)), dim3(64), 0, s,
-                     a, 1);
-  // the widest class: band DP by wavefronts (2w+1 <= 64 and <= 128), then walks
-  hipLaunchKernelGGL(k_tb_wave_dp<1>, dim3((unsigned)(n_cu * 8)), dim3(256), 0, s, a);
-  hipLaunchKernelGGL(k_tb_wave_dp<2>, dim3((unsigned)(n_cu * 8)), dim3(256), 0, s, a);
-  hipLaunchKernelGGL(k_traceback_dp<64>, dim3((unsigned)dp_blocks((const void *)k_traceback_dp<64>)), dim3(64), 0, s,
-                     a, 2);
-  const int64_t need = (a.n_alns + 63) / 64, have = n_threads / 64;
-  hipLaunchKernelGGL(k_traceback, dim3((unsigned)(need < have ? need : have)), dim3(64), 0, s, a);
-}
-
 
 // ---------------------------------------------------------------------------
 // small helpers: slow-read list, interval bases, scans

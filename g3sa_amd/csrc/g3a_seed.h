@@ -27,37 +27,9 @@
 // nearly always cover exactly min_seed_len + 1 bases, run on the lanes at
 // once and are kept up to the first that does not.
 #pragma once
-#include "g3a_dev.h"
-
-#if defined(__HIPCC__)
-#define G3A_LANE __device__ __forceinline__
-#else
-#define G3A_LANE inline
-#endif
+#include "g3a_lanes.h"
 
 namespace g3a {
-
-#if defined(__HIPCC__)
-// The lanes of a wavefront (a host test brings its own)
-struct WaveLanes {
-  static G3A_LANE uint64_t ballot(bool p) { return __ballot(p); }
-  template <class T>
-  static G3A_LANE T from(T v, int lane) { return __shfl(v, lane); }
-  template <class T>
-  static G3A_LANE T from_xor(T v, int d) { return __shfl_xor(v, d); }
-  // the wavefront's LDS stores are seen by its lanes
-  static G3A_LANE void lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  }
-  // its global stores are seen by its lanes
-  static G3A_LANE void global_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-  }
-};
-#endif
 
 // A read in LDS: 2-bit codes, 16 bases a word, first base highest (0 past
 // the end), and a mask of the bases that are N or past the end, 32 a word,
