@@ -256,17 +256,39 @@ G3A_HD ExtLaneOut ext_lane(const Opt &o, int qlen, QB qb, int tlen, TB tb, int w
     // corner rule (i+j <= 30 needs j <= i+w+1)
     const int jlim = 32 * (i0 / 32 + 1) + w + 1;
     const bool quirk = i0 >= 32 && (i0 & 31) == 0;
+    // Columns come one after another from jstart, and a strip writes a
+    // column's word only after it has read it: the words are fetched two
+    // columns ahead and the scores one, so that neither wait is in the chain.
+    auto fetch = [&](int j) { return rowbuf[(int64_t)(j < qmax ? j : qmax - 1) * rs]; };
+    uint32_t word0 = 0, word1 = 0, w0[NW];
+#pragma unroll
+    for (int k = 0; k < NW; ++k) w0[k] = 0;
+    if (jstart < qmax) {
+      word0 = fetch(jstart);
+      word1 = fetch(jstart + 1);
+#pragma unroll
+      for (int k = 0; k < NW; ++k) w0[k] = wt[(word0 >> 24) * cs + k];
+    }
+    // column j's word and scores, with those of the columns after it on their way
+    auto next_column = [&](int j, uint32_t &word, uint32_t (&wj)[NW]) {
+      word = word0;
+#pragma unroll
+      for (int k = 0; k < NW; ++k) {
+        wj[k] = w0[k];
+        w0[k] = wt[(word1 >> 24) * cs + k];
+      }
+      word0 = word1;
+      word1 = fetch(j + 2);
+    };
     // one column of the strip; kGeneral: some rule above or the band's left
     // edge may apply to a row of this column
     auto column = [&](int j, auto general_tag) {
       constexpr bool kGeneral = decltype(general_tag)::value;
-      const uint32_t word = rowbuf[(int64_t)j * rs];
+      uint32_t word, W[NW];
+      next_column(j, word, W);
       const int Ht = (int)(word & 0xfff);
       int Et = (int)((word >> 12) & 0xfff);
       const uint32_t qc = word >> 24;
-      uint32_t W[NW];
-#pragma unroll
-      for (int k = 0; k < NW; ++k) W[k] = wt[qc * cs + k];
       int hd0 = htop;
       if (kGeneral && quirk && j > i0 + w + 1) {
         const int v = h0 - oe_ins - (j - 1) * o.e_ins;
@@ -393,11 +415,10 @@ G3A_HD ExtLaneOut ext_lane(const Opt &o, int qlen, QB qb, int tlen, TB tb, int w
       uint32_t qcp;
       int e_mid, cmax_u = 0, rmin_u = R - 1;
       {
-        const uint32_t word = rowbuf[(int64_t)c0 * rs];
+        uint32_t word;
+        next_column(c0, word, wp);
         const int Ht = (int)(word & 0xfff), Et = (int)((word >> 12) & 0xfff);
         qcp = word >> 24;
-#pragma unroll
-        for (int k = 0; k < NW; ++k) wp[k] = wt[qcp * cs + k];
 #pragma unroll
         for (int r = H - 1; r >= 1; --r) {
           const int hd = hc[r - 1];
@@ -431,12 +452,10 @@ G3A_HD ExtLaneOut ext_lane(const Opt &o, int qlen, QB qb, int tlen, TB tb, int w
         fP[r] = p2(F[r], F[r + H]);
       }
       for (int c = c0 + 1; c < c1; ++c) {
-        const uint32_t word = rowbuf[(int64_t)c * rs];
+        uint32_t word, wc[NW];
+        next_column(c, word, wc);
         const int Ht = (int)(word & 0xfff), Et = (int)((word >> 12) & 0xfff);
         const uint32_t qc = word >> 24;
-        uint32_t wc[NW];
-#pragma unroll
-        for (int k = 0; k < NW; ++k) wc[k] = wt[qc * cs + k];
         // 4-row groups: upper rows' fields (column c) in the low half, lower
         // rows' (column c-1) in the high half, as signed 4-bit values
         uint32_t X[NG];
