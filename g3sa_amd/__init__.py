@@ -244,7 +244,7 @@ class Aligner:
         self._check(self.lib.g3a_set_batch_caps(self.ctx, v))
 
     def set_form(self, form: str) -> None:
-        """'plain' (one wavefront per extension task) or 'batched'."""
+        """'plain' (16 lanes per extension task) or 'batched'."""
         self._check(self.lib.g3a_set_form(self.ctx, FORMS[form]))
 
     def autotune(self) -> dict:

@@ -8,6 +8,7 @@
 // total is read back to size the next stage's buffers (grow-only, kept
 // across batches).
 #include "../../include/g3a.h"
+#include "g3a_ext_group.h"
 #include "g3a_index.h"
 #include "g3a_kernels.h"
 #include "g3a_layout.h"
@@ -151,7 +152,7 @@ struct g3a_ctx {
   std::vector<uint8_t> out_buf;
   hipEvent_t ev[8] = {};
   // single-kernel timing: k_seed, lane engine (2 sides), one-wavefront
-  // extension (2 sides or the plain form's k_extend), k_traceback
+  // extension (2 sides; the plain form's extension in all), k_traceback
   hipEvent_t kev[12] = {};
   int kev_used[6] = {0, 0, 0, 0, 0, 0};
   float kms[4] = {0, 0, 0, 0};
@@ -771,6 +772,14 @@ constexpr int kFlagSlot32 = 80;      // the flag, as an int32 index
 constexpr int kNextReadSlot32 = 82;  // k_seed's read counter (int32)
 constexpr int kChainBigSlot32 = 84;  // count of k_chain's large reads (int32)
 
+// Sides of at most this many tasks run on 16 lanes a task, larger ones on a
+// lane a task.  A lane's longest task takes 0.45 ms however few there are, and
+// a full chip of lanes 2.2 ns a task; 16 lanes take 0.1 ms and 5.5 ns a task.
+// Both sides of 150-base reads, lane against group: 568 tasks 1.28 against
+// 0.20 ms, 27,801 tasks 1.33 against 0.46 ms, 281,296 tasks about 1.7 against
+// 2.9 ms.
+constexpr int32_t kExtGroupTasks = 1 << 16;
+
 static int64_t scale(double per, int64_t n, int64_t slack) { return (int64_t)(per * (double)n) + slack; }
 
 static Caps plan_caps(const g3a_ctx *ctx, int n) {
@@ -797,15 +806,23 @@ static void free_graph(g3a_ctx *ctx) {
 
 namespace {
 
-// Buffers of the batched form's extension stage for `cap` tasks.
+// Per-task arrays of the extension stage.  The seed sort's copy and the chains
+// are dead by then, and a batch has no more tasks than seeds: the arrays lie in
+// those buffers unless the capacities grew apart.
+bool ext_shares(const Work &w, int64_t cap) {
+  return w.seeds2.bytes >= (size_t)cap * 2 * sizeof(ExtRes) && w.ch.bytes >= (size_t)cap * 12;
+}
+// Buffers of the extension stage for `cap` tasks.
 int alloc_ext(g3a_ctx *ctx, int64_t cap) {
   Work &w = *ctx->w;
+  if (!ext_shares(w, cap) &&
+      (ensure(ctx, w.ext_res[0], (size_t)cap * sizeof(ExtRes)) || ensure(ctx, w.ext_res[1], (size_t)cap * sizeof(ExtRes)) ||
+       ensure(ctx, w.ext_key, (size_t)cap * 4) || ensure(ctx, w.ext_sorted, (size_t)cap * 4) ||
+       ensure(ctx, w.ext_slow, (size_t)cap * 4)))
+    return G3A_E_HIP;
   const int lane_blocks = ctx->arena ? ctx->run_lane_blocks : ctx->n_cu * ctx->lane_blocks_per_cu;
-  return ensure(ctx, w.ext_res[0], (size_t)cap * sizeof(ExtRes)) ||
-         ensure(ctx, w.ext_res[1], (size_t)cap * sizeof(ExtRes)) || ensure(ctx, w.ext_key, (size_t)cap * 4) ||
-         ensure(ctx, w.ext_sorted, (size_t)cap * 4) || ensure(ctx, w.ext_slow, (size_t)cap * 4) ||
-         ensure(ctx, w.ext_ctr, 2 * 4 * sizeof(int32_t)) || ensure(ctx, w.ext_hist, 1024 * 4) ||
-         ensure(ctx, w.ext_rowbuf, (size_t)lane_blocks * kExtQCap * 64 * 4);
+  return ensure(ctx, w.ext_ctr, 2 * 4 * sizeof(int32_t)) || ensure(ctx, w.ext_hist, 1024 * 4) ||
+         (ctx->form != G3A_FORM_PLAIN && ensure(ctx, w.ext_rowbuf, (size_t)lane_blocks * kExtQCap * 64 * 4));
 }
 
 // Buffers of one attempt (allocation, if any, happens here and nowhere in
@@ -824,7 +841,7 @@ int alloc_batch(g3a_ctx *ctx, int n, const Caps &c) {
       alloc_paths(ctx, c.z, c.cig) || ensure(ctx, w.cig_words, (size_t)c.alns * 4 + 4) ||
       ensure(ctx, w.cig_coff, (size_t)(c.alns + 1) * 8) || ensure(ctx, w.cig_out, (size_t)c.used * 4 + 64))
     return alloc_fail(ctx);
-  if (ctx->form != G3A_FORM_PLAIN && alloc_ext(ctx, c.tasks)) return alloc_fail(ctx);
+  if (alloc_ext(ctx, c.tasks)) return alloc_fail(ctx);
   return 0;
 }
 
@@ -836,62 +853,62 @@ int alloc_batch(g3a_ctx *ctx, int n, const Caps &c) {
 static int run_extension(g3a_ctx *ctx, int64_t cap, const int64_t *n_dev, int64_t *cells, bool timed) {
   hipStream_t s = ctx->stream;
   const int32_t *stop = P<int32_t>(ctx->w->counters) + kFlagSlot32;
-  if (ctx->form == G3A_FORM_PLAIN) {
-    ExtArgs ea{};
-    ea.stop = stop;
-    ea.idx = ctx->idx;
-    ea.opt = ctx->opt;
-    ea.n_tasks = cap;
-    ea.n_dev = n_dev;
-    ea.seq = P<uint8_t>(ctx->seq);
-    ea.off = P<int32_t>(ctx->off);
-    ea.tasks = P<Task>(ctx->w->tasks);
-    ea.regs = P<Region>(ctx->w->regs);
-    ea.cells = cells;
-    if (timed) HIPCK(hipEventRecord(ctx->kev[3], s));
-    launch_extend(ea, s);
-    if (timed) HIPCK(hipEventRecord(ctx->kev[7], s));
-    ctx->kev_used[3] = timed;
-  } else if (cap > 0) {
+  if (cap > 0) {
+    const bool plain = ctx->form == G3A_FORM_PLAIN;
+    Work &w = *ctx->w;
     const int lane_blocks = ctx->arena ? ctx->run_lane_blocks : ctx->n_cu * ctx->lane_blocks_per_cu,
               wave_blocks = ctx->n_cu * ctx->wave_blocks_per_cu;
-    launch_fill_i32(P<int32_t>(ctx->w->ext_ctr), 8, 0, s);
+    const bool group_ok = ext_group_opt_ok(ctx->opt);
+    const bool shared = ext_shares(w, cap);
+    ExtRes *res[2] = {shared ? P<ExtRes>(w.seeds2) : P<ExtRes>(w.ext_res[0]),
+                      shared ? P<ExtRes>(w.seeds2) + cap : P<ExtRes>(w.ext_res[1])};
+    launch_fill_i32(P<int32_t>(w.ext_ctr), 8, 0, s);
+    if (timed && plain) HIPCK(hipEventRecord(ctx->kev[3], s));
     for (int side = 0; side < 2; ++side) {
       ExtSideArgs ea{};
       ea.stop = stop;
       ea.idx = ctx->idx;
       ea.opt = ctx->opt;
       ea.side = side;
-      ea.lane_opt_ok = ext_lane_opt_ok(ctx->opt);
+      ea.lane_opt_ok = plain ? group_ok : ext_lane_opt_ok(ctx->opt);
+      ea.group_max = !group_ok ? 0 : plain ? INT32_MAX : kExtGroupTasks;
       ea.n_tasks = cap;
       ea.n_dev = n_dev;
       ea.seq = P<uint8_t>(ctx->seq);
       ea.off = P<int32_t>(ctx->off);
-      ea.tasks = P<Task>(ctx->w->tasks);
-      ea.left = P<ExtRes>(ctx->w->ext_res[0]);
-      ea.res = P<ExtRes>(ctx->w->ext_res[side]);
-      ea.key = P<uint32_t>(ctx->w->ext_key);
-      ea.sorted = P<int32_t>(ctx->w->ext_sorted);
-      ea.slow_list = P<int32_t>(ctx->w->ext_slow);
-      ea.ctr = P<int32_t>(ctx->w->ext_ctr) + 4 * side;
-      ea.rowbuf = P<uint32_t>(ctx->w->ext_rowbuf);
+      ea.tasks = P<Task>(w.tasks);
+      ea.left = res[0];
+      ea.res = res[side];
+      ea.key = shared ? P<uint32_t>(w.ch) : P<uint32_t>(w.ext_key);
+      int32_t *sorted = shared ? P<int32_t>(w.ch) + cap : P<int32_t>(w.ext_sorted);
+      ea.sorted = sorted;
+      ea.slow_list = shared ? P<int32_t>(w.ch) + 2 * cap : P<int32_t>(w.ext_slow);
+      ea.ctr = P<int32_t>(w.ext_ctr) + 4 * side;
+      ea.rowbuf = plain ? nullptr : P<uint32_t>(w.ext_rowbuf);
       ea.cells = cells;
       launch_ext_classify(ea, s);
-      ext_sort(P<uint32_t>(ctx->w->ext_key), cap, n_dev, P<int32_t>(ctx->w->ext_hist), P<int32_t>(ctx->w->ext_sorted), s);
-      if (timed) HIPCK(hipEventRecord(ctx->kev[2 + 2 * side], s));
-      launch_ext_lane(ea, ctx->strip_rows, ctx->ext_packed, lane_blocks, s);
-      if (timed) HIPCK(hipEventRecord(ctx->kev[3 + 2 * side], s));
+      ext_sort(ea.key, cap, n_dev, P<int32_t>(w.ext_hist), sorted, s);
+      if (timed && !plain) HIPCK(hipEventRecord(ctx->kev[2 + 2 * side], s));
+      if (group_ok) launch_ext_group(ea, ctx->n_cu, s);
+      if (!plain && !(group_ok && cap <= kExtGroupTasks)) launch_ext_lane(ea, ctx->strip_rows, ctx->ext_packed, lane_blocks, s);
+      if (timed && !plain) HIPCK(hipEventRecord(ctx->kev[3 + 2 * side], s));
       launch_ext_wave(ea, wave_blocks, s);
-      if (timed) HIPCK(hipEventRecord(ctx->kev[7 + 2 * side], s));
-      ctx->kev_used[1 + side] = timed;
+      if (timed && !plain) {
+        HIPCK(hipEventRecord(ctx->kev[7 + 2 * side], s));
+        ctx->kev_used[1 + side] = timed;
+      }
+    }
+    if (timed && plain) {
+      HIPCK(hipEventRecord(ctx->kev[7], s));
+      ctx->kev_used[3] = timed;
     }
     ExtFinishArgs fa{};
     fa.stop = stop;
     fa.n_tasks = cap;
     fa.n_dev = n_dev;
     fa.tasks = P<Task>(ctx->w->tasks);
-    fa.left = P<ExtRes>(ctx->w->ext_res[0]);
-    fa.right = P<ExtRes>(ctx->w->ext_res[1]);
+    fa.left = res[0];
+    fa.right = res[1];
     fa.regs = P<Region>(ctx->w->regs);
     launch_ext_finish(fa, s);
   }

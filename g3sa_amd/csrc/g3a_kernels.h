@@ -79,28 +79,15 @@ struct CompactArgs {
   Task *tasks;
 };
 
-struct ExtArgs {
-  const int32_t *stop;  // when *stop is set the kernel returns at once (null: never)
-  DevIndex idx;
-  Opt opt;
-  int64_t n_tasks;  // capacity
-  const int64_t *n_dev;
-  const uint8_t *seq;
-  const int32_t *off;
-  const Task *tasks;
-  Region *regs;
-  int64_t *cells;
-};
-
 // Result of one side of one extension task.
 struct ExtRes {
   int32_t score, qle, tle, pad;
 };
 
-// One side (0 = left, 1 = right) of the extension stage, batched form:
-// classify -> sort lane tasks by descending query length -> lane engine
-// (persistent, chunks of 64 from a device cursor) -> one wavefront per
-// remaining task (persistent) -> finish.
+// One side (0 = left, 1 = right) of the extension stage: classify -> sort
+// lane tasks by descending query length -> lane engine (persistent, chunks of
+// 64 from a device cursor) or 16 lanes a task (chunks of 4), whichever
+// group_max says -> one wavefront per remaining task (persistent) -> finish.
 struct ExtSideArgs {
   const int32_t *stop;  // when *stop is set the kernel returns at once (null: never)
   DevIndex idx;
@@ -117,7 +104,8 @@ struct ExtSideArgs {
   uint32_t *key;          // sort key: query length of lane tasks, 0 otherwise
   const int32_t *sorted;  // lane task indices by descending key
   int32_t *slow_list;     // tasks for the one-wavefront kernel
-  int32_t *ctr;           // [0] lane tasks [1] slow tasks [2] lane chunk cursor
+  int32_t *ctr;           // [0] lane tasks [1] slow tasks [2] cursor over the lane tasks
+  int32_t group_max;      // up to this many lane tasks run on 16 lanes each
   uint32_t *rowbuf;       // kExtQCap * 64 words per lane-kernel block
   int64_t *cells;
 };
@@ -182,10 +170,10 @@ void launch_seed_slow(const SeedArgs &a, const int32_t *list, int n_list, const 
 void launch_sa_lookup(const SaArgs &a, hipStream_t s);
 void launch_chain(const ChainArgs &a, hipStream_t s);
 void launch_task_compact(const CompactArgs &a, hipStream_t s);
-void launch_extend(const ExtArgs &a, hipStream_t s);
 void launch_ext_classify(const ExtSideArgs &a, hipStream_t s);
 // packed: plain columns with two strip rows per register (16-bit lanes)
 void launch_ext_lane(const ExtSideArgs &a, int strip_rows, int packed, int n_blocks, hipStream_t s);
+void launch_ext_group(const ExtSideArgs &a, int n_cu, hipStream_t s);
 void launch_ext_wave(const ExtSideArgs &a, int n_blocks, hipStream_t s);
 void launch_ext_finish(const ExtFinishArgs &a, hipStream_t s);
 void launch_fill_i32(int32_t *p, int n, int32_t v, hipStream_t s);

@@ -6,11 +6,13 @@
 //   k_chain          wavefront per read: seed sort, chaining, chain filter,
 //                    tasks (lane 0 in global memory for the rare large read)
 //   k_task_compact   thread per read: per-read task lists -> dense task array
-//   k_extend         one wavefront per task: banded local extension, left
-//                    then right, anti-diagonal sweep over 64-row tiles
+//   k_ext_classify, k_ext_lane, k_ext_group, k_ext_wave, k_ext_finish
+//                    banded local extension, one side at a time: a lane, 16
+//                    lanes or a wavefront per task
 //   k_region_filter  thread per read
 //   k_aln_prep       thread per read: kept regions -> alignment list
 #include "g3a_dev.h"
+#include "g3a_ext_group.h"
 #include "g3a_kernels.h"
 
 #include <hip/hip_runtime.h>
@@ -984,77 +986,10 @@ __device__ ExtOut extend_wave(const Opt &o, int qlen, const uint8_t *qbuf, int t
   return r;
 }
 
-__global__ void __launch_bounds__(64) k_extend(ExtArgs a) {
-  if (a.stop && *a.stop) return;  // a capacity check before this kernel failed: the batch is redone
-  __shared__ uint8_t qbuf[kQMax];
-  __shared__ int Hbuf[2 * (kQMax + 2)], Ebuf[2 * (kQMax + 2)];
-  const int64_t t = blockIdx.x;
-  if (t >= dcount(a.n_dev, a.n_tasks)) return;
-  const Task tk = a.tasks[t];
-  const int off = a.off[tk.read], l_seq = a.off[tk.read + 1] - off;
-  const uint8_t *read = a.seq + off;
-  const int lane = threadIdx.x;
-  int64_t cells = 0;
-  Region g;
-  g.rid = tk.rid;
-  g.seedlen0 = tk.len;
-  g.secondary = 0;
-  int score;
-  // left extension: reversed read prefix against reversed reference
-  {
-    const int qlen = tk.qbeg, tlen = (int)(tk.rbeg - tk.rmax0);
-    const int h0 = tk.len * a.opt.a;
-    if (qlen > 0) {
-      for (int j = lane; j < qlen; j += 64) qbuf[j] = read[qlen - 1 - j];
-      __syncthreads();
-      const int64_t rb = tk.rbeg;
-      ExtOut e = extend_wave(
-          a.opt, qlen, qbuf, tlen, [&](int i) { return text_base(a.idx, rb - 1 - i); }, h0, a.opt.pen_clip5, Hbuf,
-          Ebuf, &cells);
-      score = e.score;
-      g.qb = tk.qbeg - e.qle;
-      g.rb = tk.rbeg - e.tle;
-      __syncthreads();
-    } else {
-      score = h0;
-      g.qb = 0;
-      g.rb = tk.rbeg;
-    }
-  }
-  // right extension
-  {
-    const int qlen = l_seq - tk.qbeg - tk.len, tlen = (int)(tk.rmax1 - tk.rbeg - tk.len);
-    const int h0 = score;
-    if (qlen > 0) {
-      for (int j = lane; j < qlen; j += 64) qbuf[j] = read[tk.qbeg + tk.len + j];
-      __syncthreads();
-      const int64_t re0 = tk.rbeg + tk.len;
-      ExtOut e = extend_wave(
-          a.opt, qlen, qbuf, tlen, [&](int i) { return text_base(a.idx, re0 + i); }, h0, a.opt.pen_clip3, Hbuf,
-          Ebuf, &cells);
-      score = e.score;
-      g.qe = tk.qbeg + tk.len + e.qle;
-      g.re = tk.rbeg + tk.len + e.tle;
-    } else {
-      g.qe = tk.qbeg + tk.len;
-      g.re = tk.rbeg + tk.len;
-    }
-  }
-  g.score = score;
-  if (lane == 0) a.regs[t] = g;
-  if (a.cells) {
-    // per-lane cell counts summed across the wave, one atomic per task
-    int64_t c = cells;
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) c += __shfl_xor(c, o);
-    if (lane == 0) atomicAdd((unsigned long long *)a.cells, (unsigned long long)c);
-  }
-}
-
 // ---------------------------------------------------------------------------
-// banded local extension, batched form: one side at a time, tasks binned by
-// query length, lane engine (g3a_ext.h) for the tasks it admits and one
-// wavefront per task (extend_wave) for the rest.
+// banded local extension: one side at a time, tasks binned by query length;
+// the tasks that the 12-bit cells admit on the lane engine (g3a_ext.h) or on
+// 16 lanes each (g3a_ext_group.h), the rest on one wavefront each (extend_wave).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int wave_min_i32(int v) {
 #pragma unroll
@@ -1155,6 +1090,7 @@ __global__ void __launch_bounds__(64) k_ext_lane(ExtSideArgs a) {
   const int lane = threadIdx.x;
   uint32_t *rb = a.rowbuf + (size_t)blockIdx.x * (kExtQCap * 64) + lane;
   const int n_lane = a.ctr[0];
+  if (n_lane <= a.group_max) return;  // k_ext_group's
   int64_t cells = 0;
   for (;;) {
     int chunk = 0;
@@ -1195,6 +1131,59 @@ __global__ void __launch_bounds__(64) k_ext_lane(ExtSideArgs a) {
       ExtRes o{r.score, r.qle, r.tle, 0};
       a.res[t] = o;
       cells += r.cells;
+    }
+  }
+  if (a.cells) {
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) cells += __shfl_xor(cells, o);
+    if (lane == 0 && cells) atomicAdd((unsigned long long *)a.cells, (unsigned long long)cells);
+  }
+}
+
+// 16 lanes per task, four tasks a wavefront, for the sides with at most
+// group_max tasks (every side in the plain form).  Three wavefronts a SIMD: at
+// four (128 VGPRs) the unrolled steps spill, 2.9 ms became 3.6 ms.
+template <bool SYM>
+__global__ void __launch_bounds__(64, 3) k_ext_group(ExtSideArgs a) {
+  if (a.stop && *a.stop) return;  // a capacity check before this kernel failed: the batch is redone
+  const int n_lane = a.ctr[0];
+  if (n_lane > a.group_max) return;  // k_ext_lane's
+  __shared__ ExtGroupStage stage[4];
+  const int lane = threadIdx.x, gl = lane & 15, gb = lane & 48;
+  int64_t cells = 0;
+  for (;;) {
+    int chunk = 0;
+    if (lane == 0) chunk = atomicAdd(a.ctr + 2, 1);
+    chunk = __shfl(chunk, 0);
+    if ((int64_t)chunk * 4 >= n_lane) break;
+    const int64_t k = (int64_t)chunk * 4 + lane / 16;
+    if (k < n_lane) {
+      const int64_t t = a.sorted[k];
+      const SideTask st = side_task(a, t);
+      const int w = ext_band_w(a.opt, st.qlen, st.end_bonus);
+      const bool left = a.side == 0;
+      const DevIndex &x = a.idx;
+      ExtGroup<WaveLanes, SYM> g{a.opt, stage + lane / 16, gl, gb};
+      const ExtGroupOut r = g.run(
+          st.qlen, [&](int j) { return (int)(left ? st.read[st.qbeg - 1 - j] : st.read[st.qend + j]); }, st.tlen,
+          [&](int i) -> uint32_t {
+            if (left) {  // row i is text position rbeg - 1 - i
+              const int64_t p = st.rbeg - 8 - i;
+              const uint64_t v = p >= 0 ? text_word(x, p) : p > -8 ? text_word(x, 0) >> (-2 * p) : 0;
+              return (uint32_t)(v >> 48);
+            }
+            return (uint32_t)(rev_sym(text_word(x, st.rend + i)) & 0xffff);
+          },
+          w, st.h0);
+      if (gl == 0) {
+        if (r.exact) {
+          a.res[t] = ExtRes{r.score, r.qle, r.tle, 0};
+        } else {
+          a.slow_list[atomicAdd(a.ctr + 1, 1)] = (int32_t)t;
+        }
+      }
+      if (a.cells && r.exact)
+        for (int i = gl; i < st.tlen; i += 16) cells += ext_row_cells(i, st.qlen, w);
     }
   }
   if (a.cells) {
@@ -1365,9 +1354,6 @@ void launch_chain(const ChainArgs &a, hipStream_t s) {
 void launch_task_compact(const CompactArgs &a, hipStream_t s) {
   if (a.n_reads) hipLaunchKernelGGL(k_task_compact, dim3(blocks(a.n_reads, 128)), dim3(128), 0, s, a);
 }
-void launch_extend(const ExtArgs &a, hipStream_t s) {
-  if (a.n_tasks) hipLaunchKernelGGL(k_extend, dim3((unsigned)a.n_tasks), dim3(64), 0, s, a);
-}
 void launch_ext_classify(const ExtSideArgs &a, hipStream_t s) {
   if (a.n_tasks) hipLaunchKernelGGL(k_ext_classify, dim3(blocks(a.n_tasks, 256 * kTilePer)), dim3(256), 0, s, a);
 }
@@ -1382,6 +1368,15 @@ void launch_ext_lane(const ExtSideArgs &a, int strip_rows, int packed, int n_blo
     k = sym ? (packed ? k_ext_lane<16, true, true> : k_ext_lane<16, true, false>)
             : (packed ? k_ext_lane<16, false, true> : k_ext_lane<16, false, false>);
   hipLaunchKernelGGL(k, dim3(n_blocks), dim3(64), 0, s, a);
+}
+void launch_ext_group(const ExtSideArgs &a, int n_cu, hipStream_t s) {
+  if (!a.n_tasks) return;
+  const bool sym = a.opt.o_del + a.opt.e_del == a.opt.o_ins + a.opt.e_ins;
+  void (*k)(ExtSideArgs) = sym ? k_ext_group<true> : k_ext_group<false>;
+  int per_cu = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, 64, 0) != hipSuccess || per_cu < 1) per_cu = 8;
+  const int64_t all = (int64_t)n_cu * per_cu, need = (a.n_tasks + 3) / 4;
+  hipLaunchKernelGGL(k, dim3((unsigned)(need < all ? need : all)), dim3(64), 0, s, a);
 }
 void launch_ext_wave(const ExtSideArgs &a, int n_blocks, hipStream_t s) {
   if (a.n_tasks) hipLaunchKernelGGL(k_ext_wave, dim3(n_blocks), dim3(64), 0, s, a);

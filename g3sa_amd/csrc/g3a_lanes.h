@@ -19,6 +19,9 @@ struct WaveLanes {
   static G3A_LANE T from(T v, int lane) { return __shfl(v, lane); }
   template <class T>
   static G3A_LANE T from_xor(T v, int d) { return __shfl_xor(v, d); }
+  // v of lane l, the same l on every lane
+  static G3A_LANE int get(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+  static G3A_LANE void lds_add(uint32_t *p, uint32_t v) { atomicAdd(p, v); }
   // v of the lane before (after) this one in the group, gl its place there;
   // the first (last) lane gets `edge`
   template <int G>

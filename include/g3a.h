@@ -176,18 +176,20 @@ void g3a_batch_out_free(g3a_batch_out *out);
 int g3a_last_stats(const g3a_ctx *ctx, float ms[6], int64_t work[6]);
 /* Device time (ms) of single kernels of the last g3a_bwa_align, from events
  * recorded on the context's stream around each launch: [0] k_seed, [1] the
- * lane extension engine (both sides; 0 in the plain form), [2] one-wavefront
- * extension (both sides, or the plain form's k_extend), [3] k_traceback.
+ * extension of the binned tasks (both sides; 0 in the plain form), [2] one-wavefront
+ * extension (both sides; the plain form's whole extension stage), [3] the
+ * traceback kernels.
  * No reference counterpart. */
 int g3a_kernel_ms(const g3a_ctx *ctx, float ms[4]);
 void g3a_destroy(g3a_ctx *ctx);
 
 /* Execution form of the extension stage.  Both forms give identical output.
- *   G3A_FORM_PLAIN    one wavefront per extension task (anti-diagonal DP)
+ *   G3A_FORM_PLAIN    16 lanes per extension task (systolic DP)
  *   G3A_FORM_BATCHED  tasks binned by query length; one task per lane in
  *                     persistent kernels pulling 64-task chunks from a
- *                     device cursor; tasks outside the lane engine's exact
- *                     domain fall back to one wavefront per task
+ *                     device cursor (16 lanes per task when there are few)
+ * In both, tasks outside the 16-bit engines' exact domain run on one
+ * wavefront per task (anti-diagonal DP).
  * No reference counterpart (the reference has one form, ksw_extend_warp2
  * under localExtending, bwa/src/aux.cu:2289-2386).  Default: BATCHED. */
 #define G3A_FORM_PLAIN 0

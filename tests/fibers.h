@@ -85,6 +85,8 @@ struct HostLanes {
     const int l = Fibers::self->cur;
     return (T)Fibers::self->meet((int64_t)v)[l ^ d];
   }
+  static int get(int v, int l) { return (int)Fibers::self->meet(v)[l]; }
+  static void lds_add(uint32_t *p, uint32_t v) { *p += v; }
   template <int G>
   static int before(int v, int edge, int gl) {
     const int64_t *b = Fibers::self->meet(v);
