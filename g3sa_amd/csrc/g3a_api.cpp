@@ -770,7 +770,8 @@ enum : int32_t {
 // counters, 40 overflow flag (int32), 41 k_seed's read counter (int32)
 constexpr int kFlagSlot32 = 80;      // the flag, as an int32 index
 constexpr int kNextReadSlot32 = 82;  // k_seed's read counter (int32)
-constexpr int kChainBigSlot32 = 84;  // count of k_chain's large reads (int32)
+constexpr int kChainBigSlot32 = 84;   // k_chain_large's counts and cursors (4 int32)
+constexpr int kRegionBigSlot32 = 88;  // k_region_large's
 
 // Sides of at most this many tasks run on 16 lanes a task, larger ones on a
 // lane a task.  A lane's longest task takes 0.45 ms however few there are, and
@@ -1023,7 +1024,7 @@ static int enqueue_batch(g3a_ctx *ctx, int n, const Caps &c, bool timed) {
   ca.serial = ctx->chain_serial;
   ca.big = P<int32_t>(w.chain_big);
   ca.n_big = P<int32_t>(w.counters) + kChainBigSlot32;
-  launch_chain(ca, s);
+  launch_chain(ca, ctx->n_cu, s);
   scan_i32(P<int32_t>(w.n_task), P<int64_t>(w.task_off), n, w.scan_tmp.p, w.scan_tmp.bytes, s);
   const int64_t *T_t = P<int64_t>(w.task_off) + n;
   launch_cap_check(T_t, c.tasks, flag, kOvTasks, s);
@@ -1035,8 +1036,9 @@ static int enqueue_batch(g3a_ctx *ctx, int n, const Caps &c, bool timed) {
   if (timed) HIPCK(hipEventRecord(ctx->ev[4], s));
   // ---- region filter, traceback, finalize
   RegionArgs ra{flag, ctx->opt, n, P<int64_t>(w.task_off), P<Region>(w.regs), P<uint8_t>(w.flag),
-                P<int32_t>(w.sec), P<int32_t>(w.n_aln)};
-  launch_region_filter(ra, s);
+                P<int32_t>(w.sec), P<int32_t>(w.n_aln), P<int32_t>(w.chain_big),
+                P<int32_t>(w.counters) + kRegionBigSlot32};
+  launch_region_filter(ra, ctx->n_cu, s);
   scan_i32(P<int32_t>(w.n_aln), P<int64_t>(w.aln_off), n, w.scan_tmp.p, w.scan_tmp.bytes, s);
   const int64_t *T_a = P<int64_t>(w.aln_off) + n;
   launch_cap_check(T_a, c.alns, flag, kOvAlns, s);

@@ -67,7 +67,7 @@ struct ChainArgs {
   Task *tasks_tmp;
   int32_t *n_task;
   int32_t *error;
-  int32_t *big, *n_big;  // reads of more than 128 seeds and their count (zero before the launch)
+  int32_t *big, *n_big;  // reads for k_chain_large; [0, 1] their counts, [2, 3] cursors (zero before the launch)
   int serial;            // 1: every read by the B-tree code on one thread (chain_one)
 };
 
@@ -128,6 +128,7 @@ struct RegionArgs {
   uint8_t *flag;
   int32_t *sec;
   int32_t *n_aln;
+  int32_t *big, *n_big;  // reads for k_region_large; [0, 1] their counts, [2, 3] cursors (zero before the launch)
 };
 
 struct AlnPrepArgs {
@@ -168,7 +169,7 @@ void launch_seed(const SeedArgs &a, int n_cu, int blocks_per_cu, int block, hipS
 void launch_seed_slow(const SeedArgs &a, const int32_t *list, int n_list, const int32_t *n_dev, int c0, Intv *scratch,
                       const int64_t *pool_off, Intv *pool, int pass, int from_scratch, hipStream_t s);
 void launch_sa_lookup(const SaArgs &a, hipStream_t s);
-void launch_chain(const ChainArgs &a, hipStream_t s);
+void launch_chain(const ChainArgs &a, int n_cu, hipStream_t s);
 void launch_task_compact(const CompactArgs &a, hipStream_t s);
 void launch_ext_classify(const ExtSideArgs &a, hipStream_t s);
 // packed: plain columns with two strip rows per register (16-bit lanes)
@@ -234,7 +235,7 @@ void launch_occ_lines(const uint32_t *W, uint64_t n, uint64_t primary, uint32_t 
 // (histogram, bin starts, scatter with per-block reservations); equal keys
 // in no fixed order.  hist: 1024 words of scratch.
 void ext_sort(const uint32_t *key, int64_t cap, const int64_t *n_dev, int32_t *hist, int32_t *out, hipStream_t s);
-void launch_region_filter(const RegionArgs &a, hipStream_t s);
+void launch_region_filter(const RegionArgs &a, int n_cu, hipStream_t s);
 void launch_aln_prep(const AlnPrepArgs &a, hipStream_t s);
 int traceback_grid_threads(int n_cu);
 int64_t traceback_pool_words(int n_threads);

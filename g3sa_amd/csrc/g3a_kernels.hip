@@ -3,21 +3,25 @@
 //
 // Stage kernels (one launch each, all on the context's stream):
 //   k_sa_lookup      thread per seed: SA interval row -> reference position
-//   k_chain          wavefront per read: seed sort, chaining, chain filter,
-//                    tasks (lane 0 in global memory for the rare large read)
+//   k_chain_thread, k_chain, k_chain_large
+//                    thread or wavefront per read: seed sort, chaining, chain
+//                    filter, tasks
 //   k_task_compact   thread per read: per-read task lists -> dense task array
 //   k_ext_classify, k_ext_lane, k_ext_group, k_ext_wave, k_ext_finish
 //                    banded local extension, one side at a time: a lane, 16
 //                    lanes or a wavefront per task
-//   k_region_filter  thread per read
+//   k_region_filter, k_region_large  thread or wavefront per read
 //   k_aln_prep       thread per read: kept regions -> alignment list
 #include "g3a_dev.h"
+#include "g3a_chain.h"
 #include "g3a_ext_group.h"
 #include "g3a_kernels.h"
+#include "g3a_region.h"
 
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 #include <rocprim/iterator/transform_iterator.hpp>
@@ -445,6 +449,18 @@ __device__ bool chain_thread(const ChainArgs &a, int r, int64_t b, int ns, const
   return true;
 }
 
+constexpr int kChainWaveSeeds = 128;  // most seeds a read may have on the wavefront path
+
+// Reads for k_chain_large: those of at most kChainMid seeds from the list's
+// front, larger ones from its back.  2^16 seeds or more, and bands beyond
+// kChainMaxW, run on this thread.
+constexpr int kChainMid = 512;
+__device__ __forceinline__ void chain_list(const ChainArgs &a, int r, int ns) {
+  if (ns >= kChainIds || a.opt.w > kChainMaxW) chain_one(a, r);
+  else if (ns <= kChainMid) a.big[atomicAdd(a.n_big, 1)] = r;
+  else a.big[a.n_reads - 1 - atomicAdd(a.n_big + 1, 1)] = r;
+}
+
 __global__ void __launch_bounds__(64) k_chain_thread(ChainArgs a) {
   if (a.stop && *a.stop) return;  // a capacity check before this kernel failed: the batch is redone
   __shared__ uint32_t lds[64 * ChainLds::kWords];
@@ -452,12 +468,12 @@ __global__ void __launch_bounds__(64) k_chain_thread(ChainArgs a) {
   if (r >= a.n_reads) return;
   const int64_t b = a.seed_off[r];
   const int ns = (int)(a.seed_off[r + 1] - b);
-  if (ns == 0 || ns > kChainThread) return;  // k_chain's
+  if (ns > kChainWaveSeeds) chain_list(a, r, ns);
+  if (ns == 0 || ns > kChainThread) return;  // k_chain's, or k_chain_large's
   const ChainLds m{lds + threadIdx.x};
-  if (!chain_thread(a, r, b, ns, m)) chain_one(a, r);
+  if (!chain_thread(a, r, b, ns, m)) chain_list(a, r, ns);
 }
 
-constexpr int kChainWaveSeeds = 128;  // most seeds a read may have on the wavefront path
 struct ChainStage {                   // one wavefront's LDS: the permutations of the sorts
   int64_t rbeg[kChainWaveSeeds];
   int32_t qbeg[kChainWaveSeeds], len[kChainWaveSeeds], rid[kChainWaveSeeds];
@@ -784,22 +800,9 @@ __device__ bool chain_wave(const ChainArgs &a, int r, int64_t b, int ns, int lan
   return true;
 }
 
-// Reads of more seeds than the wavefront path holds, listed so that k_chain
-// starts them first: each runs on one lane for far longer than a wavefront
-// read, and started in read order the last of them would be the kernel's
-// tail.
-__global__ void k_chain_big(const int32_t *stop, int n_reads, const int64_t *seed_off, int32_t *list,
-                            int32_t *n_list) {
-  if (stop && *stop) return;  // a capacity check before this kernel failed: the batch is redone
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r < n_reads && seed_off[r + 1] - seed_off[r] > kChainWaveSeeds) list[atomicAdd(n_list, 1)] = r;
-}
-
 // One wavefront per read (four a block) for reads of more than kChainThread
-// and at most kChainWaveSeeds seeds.  Wavefront g first takes the g-th
-// listed large read (chain_one on lane 0), then read g unless it is a listed
-// or a small one; reads that chain_wave hands back also run chain_one on
-// lane 0.
+// and at most kChainWaveSeeds seeds; reads that chain_wave hands back are
+// listed for k_chain_large.
 __global__ void __launch_bounds__(256) k_chain(ChainArgs a) {
   if (a.stop && *a.stop) return;  // a capacity check before this kernel failed: the batch is redone
   __shared__ ChainStage stage[4];
@@ -810,7 +813,6 @@ __global__ void __launch_bounds__(256) k_chain(ChainArgs a) {
     if (lane == 0) chain_one(a, r);
     return;
   }
-  if (r < *a.n_big && lane == 0) chain_one(a, a.big[r]);
   const int64_t b = a.seed_off[r];
   const int ns = __builtin_amdgcn_readfirstlane((int)(a.seed_off[r + 1] - b));
   bool done = true;
@@ -823,7 +825,54 @@ __global__ void __launch_bounds__(256) k_chain(ChainArgs a) {
   } else if (ns <= kChainWaveSeeds) {
     done = chain_wave<2>(a, r, b, ns, lane, stage[wv]);
   }  // else: listed
-  if (!done && lane == 0) chain_one(a, r);
+  if (!done && lane == 0) chain_list(a, r, ns);
+}
+
+// The listed reads, a wavefront each (g3a_chain.h): the B-tree itself, for
+// reads of more seeds than the wavefront's registers hold or of repeated chain
+// positions.  What bounds it is the tree descent of one seed after another.
+// On one thread the longest such read (60,000 reads of 36 to 101 bases on a
+// repeat-rich 8 Mbp text) took 70 ms, here 3.  Two classes, so that the LDS of the
+// many smaller ones (22 KB) leaves seven a compute unit; the larger have 62 KB.
+// The reads of 2^16 seeds or more and bands beyond kChainMaxW stay on a thread.
+template <bool kLarge>
+__global__ void __launch_bounds__(64) k_chain_large(ChainArgs a) {
+  if (a.stop && *a.stop) return;  // a capacity check before this kernel failed: the batch is redone
+  using Stage = std::conditional_t<kLarge, ChainStageL<2048, 290, 400, 4096>,
+                                   ChainStageL<kChainMid, kChainMid / 5 + 6, 128, kChainMid>>;
+  static_assert(sizeof(ChainTmp) == 6 * 4 && sizeof(Seed) >= 4 * 4, "a record's words lie in ch and sort_tmp");
+  // a node but the root has at least five chains: ns / 5 + 2 nodes are enough
+  static_assert(sizeof(ChainNode) * (kChainWaveSeeds / 5 + 2) + 8 <= sizeof(Task) * kChainWaveSeeds, "nodes lie in tasks_tmp");
+  __shared__ Stage st;
+  const int lane = threadIdx.x, n = a.n_big[kLarge];
+  for (;;) {
+    // The wavefront meets here: without it the compiler joins the stores of
+    // lane 0 below with its fetch of the next read, and the other lanes go
+    // round on their own.
+    WaveLanes::lds_sync();
+    int k = 0;
+    if (lane == 0) k = atomicAdd(a.n_big + 2 + kLarge, 1);
+    k = __builtin_amdgcn_readfirstlane(k);
+    if (k >= n) break;
+    const int r = a.big[kLarge ? a.n_reads - 1 - k : k];
+    const int64_t b = a.seed_off[r];
+    const int ns = (int)(a.seed_off[r + 1] - b);
+    const uintptr_t p0 = ((uintptr_t)(a.tasks_tmp + b) + 7) & ~(uintptr_t)7, p1 = (uintptr_t)(a.tasks_tmp + b + ns);
+    ChainGroup<WaveLanes, Stage> g{
+        a.idx, a.opt, &st,
+        ChainMem{(uint32_t *)(a.ch + b), (uint32_t *)(a.sort_tmp + b), a.nxt + b, a.order + b, a.tmpi + 2 * b, a.kept + b,
+                 (ChainNode *)p0, (int)((p1 - p0) / sizeof(ChainNode))}};
+    g.s = a.seeds + b;
+    g.ns = ns;
+    g.l_seq = a.off[r + 1] - a.off[r];
+    g.read = r;
+    g.lane = lane;
+    const int t = g.run(a.tasks_tmp + b);
+    if (lane == 0) {
+      if (t < 0) atomicOr(a.error, 1);  // cannot happen: reported as an error
+      a.n_task[r] = t < 0 ? 0 : t;
+    }
+  }
 }
 
 __global__ void __launch_bounds__(128) k_task_compact(CompactArgs a) {
@@ -1152,6 +1201,7 @@ __global__ void __launch_bounds__(64, 3) k_ext_group(ExtSideArgs a) {
   const int lane = threadIdx.x, gl = lane & 15, gb = lane & 48;
   int64_t cells = 0;
   for (;;) {
+    WaveLanes::lds_sync();  // the wavefront meets here, as in k_chain_large
     int chunk = 0;
     if (lane == 0) chunk = atomicAdd(a.ctr + 2, 1);
     chunk = __shfl(chunk, 0);
@@ -1304,13 +1354,50 @@ __global__ void k_fill_i32(int32_t *p, int n, int32_t v) {
 // ---------------------------------------------------------------------------
 // region filter, alignment list, traceback + finalize
 // ---------------------------------------------------------------------------
+// Reads of at most kRegionThread regions on a thread each; the others are
+// listed, those of at most kRegionMid from the list's front.
+constexpr int kRegionThread = 32, kRegionMid = 512, kRegionMax = 5120;
 __global__ void __launch_bounds__(128) k_region_filter(RegionArgs a) {
   if (a.stop && *a.stop) return;  // a capacity check before this kernel failed: the batch is redone
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= a.n_reads) return;
   const int64_t b = a.task_off[r];
   const int n = (int)(a.task_off[r + 1] - b);
+  if (n > kRegionThread) {  // k_region_large's
+    if (n <= kRegionMid) a.big[atomicAdd(a.n_big, 1)] = r;
+    else a.big[a.n_reads - 1 - atomicAdd(a.n_big + 1, 1)] = r;
+    return;
+  }
   a.n_aln[r] = n ? region_filter(a.opt, a.regs + b, n, a.flag + b, a.sec + b) : 0;
+}
+// The reads of more than kRegionThread regions, a wavefront each
+// (g3a_region.h).  What bounds it is LDS latency, a pair of regions a lane; on
+// one thread the longest read (60,000 reads of 36 to 101 bases on a repeat-rich
+// 8 Mbp text) took 30 ms, here 1.  Two classes, as in k_chain_large (15 KB and 154 KB
+// of LDS); more than kRegionMax regions stay on a thread.
+template <bool kLarge>
+__global__ void __launch_bounds__(64) k_region_large(RegionArgs a) {
+  if (a.stop && *a.stop) return;  // a capacity check before this kernel failed: the batch is redone
+  using Stage = RegionStage<kLarge ? kRegionMax : kRegionMid>;
+  __shared__ Stage st;
+  const int lane = threadIdx.x, n_list = a.n_big[kLarge];
+  for (;;) {
+    WaveLanes::lds_sync();  // the wavefront meets here, as in k_chain_large
+    int k = 0;
+    if (lane == 0) k = atomicAdd(a.n_big + 2 + kLarge, 1);
+    k = __builtin_amdgcn_readfirstlane(k);
+    if (k >= n_list) break;
+    const int r = a.big[kLarge ? a.n_reads - 1 - k : k];
+    const int64_t b = a.task_off[r];
+    const int n = (int)(a.task_off[r + 1] - b);
+    if (n <= Stage::kMax) {
+      RegionGroup<WaveLanes, Stage> g{a.opt, &st, lane};
+      const int m = g.run(a.regs + b, n);
+      if (lane == 0) a.n_aln[r] = m;
+    } else if (lane == 0) {
+      a.n_aln[r] = region_filter(a.opt, a.regs + b, n, a.flag + b, a.sec + b);
+    }
+  }
 }
 
 __global__ void __launch_bounds__(128) k_aln_prep(AlnPrepArgs a) {
@@ -1340,16 +1427,25 @@ static inline unsigned blocks(int64_t n, int bs) { return (unsigned)((n + bs - 1
 void launch_sa_lookup(const SaArgs &a, hipStream_t s) {
   if (a.total) hipLaunchKernelGGL(k_sa_lookup, dim3(blocks(a.total, 256)), dim3(256), 0, s, a);
 }
-void launch_chain(const ChainArgs &a, hipStream_t s) {
+// blocks of a persistent grid of one-wavefront blocks for at most n items
+static unsigned persistent(const void *k, int n_cu, int64_t n) {
+  int per_cu = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, 64, 0) != hipSuccess || per_cu < 1) per_cu = 1;
+  const int64_t all = (int64_t)n_cu * per_cu;
+  return (unsigned)(n < all ? n : all);
+}
+void launch_chain(const ChainArgs &a, int n_cu, hipStream_t s) {
   if (!a.n_reads) return;
   if (a.serial) {
     hipLaunchKernelGGL(k_chain, dim3(blocks(a.n_reads, 4)), dim3(256), 0, s, a);
     return;
   }
-  hipLaunchKernelGGL(k_chain_big, dim3(blocks(a.n_reads, 256)), dim3(256), 0, s, a.stop, a.n_reads, a.seed_off,
-                     a.big, a.n_big);
   hipLaunchKernelGGL(k_chain_thread, dim3(blocks(a.n_reads, 64)), dim3(64), 0, s, a);
   hipLaunchKernelGGL(k_chain, dim3(blocks(a.n_reads, 4)), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(k_chain_large<true>, dim3(persistent((const void *)k_chain_large<true>, n_cu, a.n_reads)), dim3(64), 0,
+                     s, a);
+  hipLaunchKernelGGL(k_chain_large<false>, dim3(persistent((const void *)k_chain_large<false>, n_cu, a.n_reads)), dim3(64),
+                     0, s, a);
 }
 void launch_task_compact(const CompactArgs &a, hipStream_t s) {
   if (a.n_reads) hipLaunchKernelGGL(k_task_compact, dim3(blocks(a.n_reads, 128)), dim3(128), 0, s, a);
@@ -1387,8 +1483,13 @@ void launch_ext_finish(const ExtFinishArgs &a, hipStream_t s) {
 void launch_fill_i32(int32_t *p, int n, int32_t v, hipStream_t s) {
   if (n) hipLaunchKernelGGL(k_fill_i32, dim3(blocks(n, 256)), dim3(256), 0, s, p, n, v);
 }
-void launch_region_filter(const RegionArgs &a, hipStream_t s) {
-  if (a.n_reads) hipLaunchKernelGGL(k_region_filter, dim3(blocks(a.n_reads, 128)), dim3(128), 0, s, a);
+void launch_region_filter(const RegionArgs &a, int n_cu, hipStream_t s) {
+  if (!a.n_reads) return;
+  hipLaunchKernelGGL(k_region_filter, dim3(blocks(a.n_reads, 128)), dim3(128), 0, s, a);
+  hipLaunchKernelGGL(k_region_large<true>, dim3(persistent((const void *)k_region_large<true>, n_cu, a.n_reads)), dim3(64),
+                     0, s, a);
+  hipLaunchKernelGGL(k_region_large<false>, dim3(persistent((const void *)k_region_large<false>, n_cu, a.n_reads)), dim3(64),
+                     0, s, a);
 }
 void launch_aln_prep(const AlnPrepArgs &a, hipStream_t s) {
   if (a.n_reads) hipLaunchKernelGGL(k_aln_prep, dim3(blocks(a.n_reads, 128)), dim3(128), 0, s, a);
