@@ -8,6 +8,7 @@
 // total is read back to size the next stage's buffers (grow-only, kept
 // across batches).
 #include "../../include/g3a.h"
+#include "g3a_copy.h"
 #include "g3a_ext_group.h"
 #include "g3a_index.h"
 #include "g3a_kernels.h"
@@ -148,7 +149,8 @@ struct g3a_ctx {
   int64_t *pinned = nullptr;
   static constexpr size_t kStage = (size_t)16 << 20;
   uint8_t *stage[2] = {nullptr, nullptr};
-  hipEvent_t stage_ev[2] = {};
+  hipEvent_t stage_ev[CopyCrew::kSlots] = {};
+  CopyCrew crew;  // the threads that copy through the staging slots
   std::vector<uint8_t> out_buf;
   hipEvent_t ev[8] = {};
   // single-kernel timing: k_seed, lane engine (2 sides), one-wavefront
@@ -227,10 +229,32 @@ int ensure(g3a_ctx *ctx, DevBuf &b, size_t bytes) {
   return 0;
 }
 
-// Host <-> device copies of pageable memory through two page-locked
-// staging slots: the CPU copy into (or out of) one slot overlaps the DMA of
-// the other.  Both end with the stream synchronized.
+// Host <-> device copies of pageable memory through page-locked staging
+// slots: the CPU copies into (or out of) some slots overlap the DMA of others.
+// All end with the stream synchronized.  From kCrewBytes on several threads
+// copy (g3a_copy.h): below, waking them costs what they save.
+constexpr size_t kCrewBytes = (size_t)2 << 20, kCrewChunk = g3a_ctx::kStage * 2 / CopyCrew::kSlots;
+uint8_t *crew_slot(g3a_ctx *ctx, size_t i) {
+  const size_t k = i % CopyCrew::kSlots, per = CopyCrew::kSlots / 2;
+  return ctx->stage[k / per] + k % per * kCrewChunk;
+}
 int stage_h2d(g3a_ctx *ctx, void *dev, const void *src, size_t bytes) {
+  if (bytes >= kCrewBytes && ctx->crew.ready()) {
+    const int rc = ctx->crew.in(
+        (const uint8_t *)src, bytes, kCrewChunk, [&](size_t i) { return crew_slot(ctx, i); },
+        [&](size_t i, size_t at, size_t m) -> int {
+          HIPCK(hipMemcpyAsync((uint8_t *)dev + at, crew_slot(ctx, i), m, hipMemcpyHostToDevice, ctx->stream));
+          HIPCK(hipEventRecord(ctx->stage_ev[i % CopyCrew::kSlots], ctx->stream));
+          return 0;
+        },
+        [&](size_t i) -> int {
+          HIPCK(hipEventSynchronize(ctx->stage_ev[i % CopyCrew::kSlots]));
+          return 0;
+        });
+    if (rc) return rc;
+    HIPCK(hipStreamSynchronize(ctx->stream));
+    return 0;
+  }
   const size_t K = g3a_ctx::kStage;
   for (size_t c = 0, i = 0; c < bytes; c += K, ++i) {
     const int k = (int)(i & 1);
@@ -245,6 +269,22 @@ int stage_h2d(g3a_ctx *ctx, void *dev, const void *src, size_t bytes) {
 }
 
 int stage_d2h(g3a_ctx *ctx, void *dst, const void *dev, size_t bytes) {
+  if (bytes >= kCrewBytes && ctx->crew.ready()) {
+    const int rc = ctx->crew.out(
+        (uint8_t *)dst, bytes, kCrewChunk, [&](size_t i) { return crew_slot(ctx, i); },
+        [&](size_t i, size_t at, size_t m) -> int {
+          HIPCK(hipMemcpyAsync(crew_slot(ctx, i), (const uint8_t *)dev + at, m, hipMemcpyDeviceToHost, ctx->stream));
+          HIPCK(hipEventRecord(ctx->stage_ev[i % CopyCrew::kSlots], ctx->stream));
+          return 0;
+        },
+        [&](size_t i) -> int {
+          HIPCK(hipEventSynchronize(ctx->stage_ev[i % CopyCrew::kSlots]));
+          return 0;
+        });
+    if (rc) return rc;
+    HIPCK(hipStreamSynchronize(ctx->stream));
+    return 0;
+  }
   const size_t K = g3a_ctx::kStage, n = (bytes + K - 1) / K;
   auto issue = [&](size_t i) -> int {
     const size_t c = i * K, m = bytes - c < K ? bytes - c : K;
@@ -303,10 +343,10 @@ int init_runtime(g3a_ctx *ctx) {
     ctx->n_cu = 256;
   if (hipHostMalloc((void **)&ctx->pinned, 64 * sizeof(int64_t), hipHostMallocDefault) != hipSuccess ||
       hipHostMalloc((void **)&ctx->stage[0], g3a_ctx::kStage, hipHostMallocDefault) != hipSuccess ||
-      hipHostMalloc((void **)&ctx->stage[1], g3a_ctx::kStage, hipHostMallocDefault) != hipSuccess ||
-      hipEventCreateWithFlags(&ctx->stage_ev[0], hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&ctx->stage_ev[1], hipEventDisableTiming) != hipSuccess)
+      hipHostMalloc((void **)&ctx->stage[1], g3a_ctx::kStage, hipHostMallocDefault) != hipSuccess)
     return G3A_E_HIP;
+  for (auto &ev : ctx->stage_ev)
+    if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) return G3A_E_HIP;
   // the allocation-free entry point's scratch array on this device (set up
   // here, with the device current)
   if (scratch_address(ctx->device, &ctx->scratch) != hipSuccess) return G3A_E_HIP;
@@ -1879,10 +1919,10 @@ void g3a_destroy(g3a_ctx *ctx) {
   for (auto &ev : ctx->kev)
     if (ev) hipEventDestroy(ev);
   if (ctx->pinned) hipHostFree(ctx->pinned);
-  for (int k = 0; k < 2; ++k) {
-    if (ctx->stage[k]) hipHostFree(ctx->stage[k]);
-    if (ctx->stage_ev[k]) hipEventDestroy(ctx->stage_ev[k]);
-  }
+  for (uint8_t *p : ctx->stage)
+    if (p) hipHostFree(p);
+  for (auto &ev : ctx->stage_ev)
+    if (ev) hipEventDestroy(ev);
   if (ctx->stream) hipStreamDestroy(ctx->stream);
   delete ctx;
 }
