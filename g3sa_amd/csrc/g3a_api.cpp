@@ -820,6 +820,8 @@ constexpr int kRegionBigSlot32 = 88;  // k_region_large's
 // 0.20 ms, 27,801 tasks 1.33 against 0.46 ms, 281,296 tasks about 1.7 against
 // 2.9 ms.
 constexpr int32_t kExtGroupTasks = 1 << 16;
+// 568 tasks 0.20 ms either way; 11,517 sorted 0.35, unsorted 0.37 ms.
+constexpr int64_t kExtUnsorted = 1 << 12;
 
 static int64_t scale(double per, int64_t n, int64_t slack) { return (int64_t)(per * (double)n) + slack; }
 
@@ -927,8 +929,11 @@ static int run_extension(g3a_ctx *ctx, int64_t cap, const int64_t *n_dev, int64_
       ea.ctr = P<int32_t>(w.ext_ctr) + 4 * side;
       ea.rowbuf = plain ? nullptr : P<uint32_t>(w.ext_rowbuf);
       ea.cells = cells;
+      // few enough tasks for every group to start at once: their order is
+      // nothing to gain by, and sorting them takes four launches
+      if (group_ok && cap <= kExtUnsorted) ea.unsorted = sorted;
       launch_ext_classify(ea, s);
-      ext_sort(ea.key, cap, n_dev, P<int32_t>(w.ext_hist), sorted, s);
+      if (!ea.unsorted) ext_sort(ea.key, cap, n_dev, P<int32_t>(w.ext_hist), sorted, s);
       if (timed && !plain) HIPCK(hipEventRecord(ctx->kev[2 + 2 * side], s));
       if (group_ok) launch_ext_group(ea, ctx->n_cu, s);
       if (!plain && !(group_ok && cap <= kExtGroupTasks)) launch_ext_lane(ea, ctx->strip_rows, ctx->ext_packed, lane_blocks, s);
@@ -1002,7 +1007,6 @@ static int enqueue_batch(g3a_ctx *ctx, int n, const Caps &c, bool timed) {
   launch_collect_slow(n, P<int32_t>(w.slow), P<int32_t>(w.slow_list), n_slow_dev, P<int64_t>(w.intv_base), kSlotCap, s);
   // reads whose lists outgrew the fast path: counts (pass 0), pool offsets,
   // then the intervals (pass 1), all for the device's count of them
-  launch_cap_check32(n_slow_dev, c.slow, flag, kOvSlow, s);
   {
     const int chunk = ctx->run_slow_chunk < c.slow ? ctx->run_slow_chunk : c.slow;
     const int32_t *list = P<int32_t>(w.slow_list);
@@ -1010,23 +1014,21 @@ static int enqueue_batch(g3a_ctx *ctx, int n, const Caps &c, bool timed) {
       const int m = c.slow - c0 < chunk ? c.slow - c0 : chunk;
       launch_seed_slow(sa, list + c0, m, n_slow_dev, c0, P<Intv>(w.slow_scratch), nullptr, nullptr, 0, 0, s);
     }
-    launch_gather_slow_counts(c.slow, n_slow_dev, list, P<int32_t>(w.n_intv), P<int64_t>(w.slow_n), s);
-    scan_i64(P<int64_t>(w.slow_n), P<int64_t>(w.slow_off), c.slow, w.scan_tmp.p, w.scan_tmp.bytes, s);
-    launch_cap_check(P<int64_t>(w.slow_off) + c.slow, c.pool, flag, kOvPool, s);
+    scan_slow(c.slow, n_slow_dev, list, P<int32_t>(w.n_intv), P<int64_t>(w.slow_n), P<int64_t>(w.slow_off),
+              CapCheck{c.pool, flag, kOvPool}, (int64_t)fast_entries, P<int64_t>(w.intv_base), kOvSlow, w.scan_tmp.p,
+              w.scan_tmp.bytes, s);
     Intv *pool_base = P<Intv>(w.intv) + fast_entries;
     for (int c0 = 0; c0 < c.slow; c0 += chunk) {
       const int m = c.slow - c0 < chunk ? c.slow - c0 : chunk;
       launch_seed_slow(sa, list + c0, m, n_slow_dev, c0, P<Intv>(w.slow_scratch), P<int64_t>(w.slow_off) + c0,
                        pool_base, 1, c.slow <= chunk, s);
     }
-    launch_set_slow_base(c.slow, n_slow_dev, list, P<int64_t>(w.slow_off), (int64_t)fast_entries,
-                         P<int64_t>(w.intv_base), s);
   }
   if (timed) HIPCK(hipEventRecord(ctx->ev[1], s));
   // ---- SA lookup (the seeds are sorted by the chaining kernel)
-  scan_i64(P<int64_t>(w.n_seed), P<int64_t>(w.seed_off), n, w.scan_tmp.p, w.scan_tmp.bytes, s);
+  scan_i64(P<int64_t>(w.n_seed), P<int64_t>(w.seed_off), n, w.scan_tmp.p, w.scan_tmp.bytes, s,
+           CapCheck{c.seeds, flag, kOvSeeds});
   const int64_t *T_s = P<int64_t>(w.seed_off) + n;
-  launch_cap_check(T_s, c.seeds, flag, kOvSeeds, s);
   SaArgs la{};
   la.stop = flag;
   la.idx = ctx->idx;
@@ -1065,9 +1067,9 @@ static int enqueue_batch(g3a_ctx *ctx, int n, const Caps &c, bool timed) {
   ca.big = P<int32_t>(w.chain_big);
   ca.n_big = P<int32_t>(w.counters) + kChainBigSlot32;
   launch_chain(ca, ctx->n_cu, s);
-  scan_i32(P<int32_t>(w.n_task), P<int64_t>(w.task_off), n, w.scan_tmp.p, w.scan_tmp.bytes, s);
+  scan_i32(P<int32_t>(w.n_task), P<int64_t>(w.task_off), n, w.scan_tmp.p, w.scan_tmp.bytes, s,
+           CapCheck{c.tasks, flag, kOvTasks});
   const int64_t *T_t = P<int64_t>(w.task_off) + n;
-  launch_cap_check(T_t, c.tasks, flag, kOvTasks, s);
   CompactArgs cp{flag, n, P<int64_t>(w.seed_off), P<int64_t>(w.task_off), P<Task>(w.tasks_tmp), P<Task>(w.tasks)};
   launch_task_compact(cp, s);
   if (timed) HIPCK(hipEventRecord(ctx->ev[3], s));
@@ -1079,20 +1081,15 @@ static int enqueue_batch(g3a_ctx *ctx, int n, const Caps &c, bool timed) {
                 P<int32_t>(w.sec), P<int32_t>(w.n_aln), P<int32_t>(w.chain_big),
                 P<int32_t>(w.counters) + kRegionBigSlot32};
   launch_region_filter(ra, ctx->n_cu, s);
-  scan_i32(P<int32_t>(w.n_aln), P<int64_t>(w.aln_off), n, w.scan_tmp.p, w.scan_tmp.bytes, s);
+  scan_i32(P<int32_t>(w.n_aln), P<int64_t>(w.aln_off), n, w.scan_tmp.p, w.scan_tmp.bytes, s,
+           CapCheck{c.alns, flag, kOvAlns});
   const int64_t *T_a = P<int64_t>(w.aln_off) + n;
-  launch_cap_check(T_a, c.alns, flag, kOvAlns, s);
   AlnPrepArgs ap{flag, ctx->opt, n, P<int64_t>(w.task_off), P<int64_t>(w.aln_off), P<Region>(w.regs),
                  P<Region>(w.aln_reg), P<int32_t>(w.aln_read), P<int32_t>(w.aln_rank),
                  P<int64_t>(w.z_size), P<int64_t>(w.cig_size)};
   launch_aln_prep(ap, s);
-  // sizes past the alignments count nothing in the scans over the capacity
-  launch_zero_tail(P<int64_t>(w.z_size), c.alns, T_a, s);
-  launch_zero_tail(P<int64_t>(w.cig_size), c.alns, T_a, s);
-  scan_i64(P<int64_t>(w.z_size), P<int64_t>(w.z_off), c.alns, w.scan_tmp.p, w.scan_tmp.bytes, s);
-  scan_i64(P<int64_t>(w.cig_size), P<int64_t>(w.cig_off), c.alns, w.scan_tmp.p, w.scan_tmp.bytes, s);
-  launch_cap_check(P<int64_t>(w.z_off) + c.alns, c.z, flag, kOvZ, s);
-  launch_cap_check(P<int64_t>(w.cig_off) + c.alns, c.cig, flag, kOvCig, s);
+  scan_paths(P<int64_t>(w.z_size), P<int64_t>(w.z_off), CapCheck{c.z, flag, kOvZ}, P<int64_t>(w.cig_size),
+             P<int64_t>(w.cig_off), CapCheck{c.cig, flag, kOvCig}, c.alns, T_a, w.scan_tmp.p, w.scan_tmp.bytes, s);
   TbArgs tb{};
   tb.stop = flag;
   tb.idx = ctx->idx;
@@ -1117,9 +1114,8 @@ static int enqueue_batch(g3a_ctx *ctx, int n, const Caps &c, bool timed) {
   if (timed) HIPCK(hipEventRecord(ctx->kev[11], s));
   ctx->kev_used[5] = timed;
   // CIGARs packed to the words used, for the copy to the host
-  launch_cig_words(P<Aln>(w.alns), c.alns, T_a, P<int32_t>(w.cig_words), s);
-  scan_i32(P<int32_t>(w.cig_words), P<int64_t>(w.cig_coff), c.alns, w.scan_tmp.p, w.scan_tmp.bytes, s);
-  launch_cap_check(P<int64_t>(w.cig_coff) + c.alns, c.used, flag, kOvUsed, s);
+  scan_cig_words(P<Aln>(w.alns), c.alns, T_a, P<int32_t>(w.cig_words), P<int64_t>(w.cig_coff),
+                 CapCheck{c.used, flag, kOvUsed}, w.scan_tmp.p, w.scan_tmp.bytes, s);
   launch_cig_gather(P<Aln>(w.alns), c.alns, T_a, flag, P<int64_t>(w.cig_coff), P<uint32_t>(w.cigar),
                     P<uint32_t>(w.cig_out), s);
   // the totals, for the one read-back of the batch

@@ -102,6 +102,7 @@ struct ExtSideArgs {
   const ExtRes *left;     // left results: h0 of the right side
   ExtRes *res;            // this side's results
   uint32_t *key;          // sort key: query length of lane tasks, 0 otherwise
+  int32_t *unsorted;      // lane task indices as classified, instead of keys (null: keys)
   const int32_t *sorted;  // lane task indices by descending key
   int32_t *slow_list;     // tasks for the one-wavefront kernel
   int32_t *ctr;           // [0] lane tasks [1] slow tasks [2] cursor over the lane tasks
@@ -260,8 +261,27 @@ void launch_gather_totals(const Gather16 &g, int k, int64_t *dst, hipStream_t s)
 
 // exclusive scans (rocPRIM) over int32 or int64 counts into int64 offsets;
 // out has n+1 entries, out[n] = total
-void scan_i32(const int32_t *in, int64_t *out, int64_t n, void *tmp, size_t tmp_bytes, hipStream_t s);
-void scan_i64(const int64_t *in, int64_t *out, int64_t n, void *tmp, size_t tmp_bytes, hipStream_t s);
+// A total over cap sets *flag to bit, unless an earlier check set it (flag
+// null: no check).
+struct CapCheck {
+  int64_t cap = 0;
+  int32_t *flag = nullptr;
+  int32_t bit = 0;
+};
+void scan_i32(const int32_t *in, int64_t *out, int64_t n, void *tmp, size_t tmp_bytes, hipStream_t s,
+              const CapCheck &ck = CapCheck());
+void scan_i64(const int64_t *in, int64_t *out, int64_t n, void *tmp, size_t tmp_bytes, hipStream_t s,
+              const CapCheck &ck = CapCheck());
+// direction bytes and CIGAR words of the first *n_dev alignments
+void scan_paths(int64_t *z, int64_t *z_off, const CapCheck &ck_z, int64_t *cig, int64_t *cig_off, const CapCheck &ck_cig,
+                int64_t cap, const int64_t *n_dev, void *tmp, size_t tmp_bytes, hipStream_t s);
+void scan_cig_words(const Aln *alns, int64_t cap, const int64_t *n_dev, int32_t *words, int64_t *out, const CapCheck &ck,
+                    void *tmp, size_t tmp_bytes, hipStream_t s);
+// between the slow reads' passes: their pool offsets and the places of their
+// intervals; more of them than cap sets `bit`
+void scan_slow(int cap, const int32_t *n_dev, const int32_t *list, const int32_t *n_intv, int64_t *counts, int64_t *out,
+               const CapCheck &ck, int64_t base, int64_t *intv_base, int32_t bit, void *tmp, size_t tmp_bytes,
+               hipStream_t s);
 size_t scan_tmp_bytes(int64_t n);
 void launch_seed_keys(const uint8_t *seq, const int32_t *off, int n, uint32_t *key, int32_t *idx, hipStream_t s);
 size_t seed_sort_tmp_bytes(int64_t n);

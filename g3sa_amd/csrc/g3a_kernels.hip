@@ -1097,7 +1097,7 @@ __global__ void __launch_bounds__(256) k_ext_classify(ExtSideArgs a) {
   __syncthreads();
   const int64_t tile = (int64_t)blockIdx.x * (256 * kTilePer);
   const int64_t n = dcount(a.n_dev, a.n_tasks);
-  int n_lane = 0, slow_at[kTilePer];
+  int n_lane = 0, slow_at[kTilePer], lane_at[kTilePer];
 #pragma unroll
   for (int i = 0; i < kTilePer; ++i) {
     const int64_t t = tile + i * 256 + threadIdx.x;
@@ -1115,20 +1115,28 @@ __global__ void __launch_bounds__(256) k_ext_classify(ExtSideArgs a) {
       }
       if (lane) key = (uint32_t)st.qlen;
     }
-    if (t < a.n_tasks) a.key[t] = key;
+    if (a.unsorted) {
+      lane_at[i] = lane ? atomicAdd(&cnt[0], 1) : -1;
+    } else if (t < a.n_tasks) {
+      a.key[t] = key;
+    }
     n_lane += lane;
     slow_at[i] = slow ? atomicAdd(&cnt[1], 1) : -1;
   }
-  if (n_lane) atomicAdd(&cnt[0], n_lane);
+  if (n_lane && !a.unsorted) atomicAdd(&cnt[0], n_lane);
   __syncthreads();
   if (threadIdx.x == 0) {
-    if (cnt[0]) atomicAdd(a.ctr, cnt[0]);
+    base[0] = cnt[0] ? atomicAdd(a.ctr, cnt[0]) : 0;
     base[1] = cnt[1] ? atomicAdd(a.ctr + 1, cnt[1]) : 0;
   }
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < kTilePer; ++i)
     if (slow_at[i] >= 0) a.slow_list[base[1] + slow_at[i]] = (int32_t)(tile + i * 256 + threadIdx.x);
+  if (a.unsorted)
+#pragma unroll
+    for (int i = 0; i < kTilePer; ++i)
+      if (lane_at[i] >= 0) a.unsorted[base[0] + lane_at[i]] = (int32_t)(tile + i * 256 + threadIdx.x);
 }
 
 template <int R, bool SYM, bool PK>
@@ -1629,15 +1637,139 @@ size_t scan_tmp_bytes(int64_t n) {
                           rocprim::plus<int64_t>());
   return (a > b ? a : b) + 256;
 }
-void scan_i64(const int64_t *in, int64_t *out, int64_t n, void *tmp, size_t tmp_bytes, hipStream_t s) {
-  hipLaunchKernelGGL(k_zero_first, dim3(1), dim3(1), 0, s, out);
-  if (n > 0) rocprim::inclusive_scan(tmp, tmp_bytes, in, out + 1, (size_t)n, rocprim::plus<int64_t>(), s);
+// What a scan reads
+struct ScanI64 {
+  const int64_t *p;
+  __device__ int64_t operator()(int i) const { return p[i]; }
+};
+struct ScanI32 {
+  const int32_t *p;
+  __device__ int64_t operator()(int i) const { return p[i]; }
+};
+struct ScanHead {  // the first *n_dev of p, then zeros
+  const int64_t *p, *n_dev;
+  __device__ int64_t operator()(int i) const { return i < *n_dev ? p[i] : 0; }
+};
+struct ScanSlow {  // the interval counts of the listed reads
+  const int32_t *list, *n_intv, *n_dev;
+  __device__ int64_t operator()(int i) const { return i < *n_dev ? n_intv[list[i]] : 0; }
+};
+struct ScanWords {  // CIGAR words of the first *n_dev alignments
+  const Aln *alns;
+  const int64_t *n_dev;
+  __device__ int64_t operator()(int i) const { return i < *n_dev ? alns[i].n_cigar + alns[i].n_core : 0; }
+};
+// Prefix sums of up to kScanSmall numbers in one block: out[i] = the sum of
+// the first i, out[n] checked against ck.  A short scan is all launches: the
+// library's takes two, with the zero before it, the zeros past the count and
+// the check after it three more, at 4 to 5 us each; this one 4 to 8 us.  A
+// batch of 200 reads has six.
+constexpr int kScanSmall = 1 << 14, kScanThreads = 1024;
+template <class F>
+__device__ __forceinline__ void scan_block(F f, int n, int64_t *out, const CapCheck &ck) {
+  __shared__ int64_t wave_sum[kScanThreads / 64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, per = (n + kScanThreads - 1) / kScanThreads;
+  const int i0 = threadIdx.x * per, i1 = i0 + per < n ? i0 + per : n;
+  int64_t v[kScanSmall / kScanThreads], sum = 0;
+#pragma unroll
+  for (int k = 0; k < kScanSmall / kScanThreads; ++k) {
+    v[k] = i0 + k < i1 ? f(i0 + k) : 0;
+    sum += v[k];
+  }
+  int64_t incl = sum;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int64_t u = __shfl_up(incl, d);
+    incl += lane >= d ? u : 0;
+  }
+  if (lane == 63) wave_sum[wv] = incl;
+  __syncthreads();
+  int64_t at = incl - sum, total = 0;
+#pragma unroll
+  for (int w = 0; w < kScanThreads / 64; ++w) {
+    at += w < wv ? wave_sum[w] : 0;
+    total += wave_sum[w];
+  }
+#pragma unroll
+  for (int k = 0; k < kScanSmall / kScanThreads; ++k) {
+    at += v[k];
+    if (i0 + k < i1) out[i0 + k + 1] = at;
+  }
+  if (threadIdx.x == 0) {
+    out[0] = 0;
+    if (ck.flag && total > ck.cap && !*ck.flag) *ck.flag = ck.bit;  // the first check that fails, as in k_cap_check
+  }
 }
-void scan_i32(const int32_t *in, int64_t *out, int64_t n, void *tmp, size_t tmp_bytes, hipStream_t s) {
+template <class F>
+__global__ void __launch_bounds__(kScanThreads) k_scan_small(F f, int n, int64_t *out, CapCheck ck) {
+  scan_block(f, n, out, ck);
+}
+// two of them, one after the other
+template <class F>
+__global__ void __launch_bounds__(kScanThreads) k_scan_small2(F f0, F f1, int n, int64_t *out0, int64_t *out1, CapCheck ck0,
+                                                              CapCheck ck1) {
+  scan_block(f0, n, out0, ck0);
+  __syncthreads();
+  scan_block(f1, n, out1, ck1);
+}
+// The pool offsets of the listed slow reads, and where their intervals start
+__global__ void __launch_bounds__(kScanThreads) k_slow_offsets(ScanSlow f, int cap, int64_t *out, CapCheck ck, int64_t base,
+                                                               int64_t *intv_base, int32_t bit) {
+  if (threadIdx.x == 0 && *f.n_dev > cap && !*ck.flag) *ck.flag = bit;
+  scan_block(f, cap, out, ck);
+  __syncthreads();
+  for (int t = threadIdx.x; t < cap && t < *f.n_dev; t += kScanThreads) intv_base[f.list[t]] = base + out[t];
+}
+template <class F>
+static void scan_small(F f, int64_t n, int64_t *out, const CapCheck &ck, hipStream_t s) {
+  hipLaunchKernelGGL(k_scan_small<F>, dim3(1), dim3(kScanThreads), 0, s, f, (int)n, out, ck);
+}
+void scan_i64(const int64_t *in, int64_t *out, int64_t n, void *tmp, size_t tmp_bytes, hipStream_t s, const CapCheck &ck) {
+  if (n <= kScanSmall) return scan_small(ScanI64{in}, n, out, ck, s);
   hipLaunchKernelGGL(k_zero_first, dim3(1), dim3(1), 0, s, out);
-  if (n > 0)
-    rocprim::inclusive_scan(tmp, tmp_bytes, rocprim::make_transform_iterator(in, WidenI32()), out + 1, (size_t)n,
-                            rocprim::plus<int64_t>(), s);
+  rocprim::inclusive_scan(tmp, tmp_bytes, in, out + 1, (size_t)n, rocprim::plus<int64_t>(), s);
+  if (ck.flag) launch_cap_check(out + n, ck.cap, ck.flag, ck.bit, s);
+}
+void scan_i32(const int32_t *in, int64_t *out, int64_t n, void *tmp, size_t tmp_bytes, hipStream_t s, const CapCheck &ck) {
+  if (n <= kScanSmall) return scan_small(ScanI32{in}, n, out, ck, s);
+  hipLaunchKernelGGL(k_zero_first, dim3(1), dim3(1), 0, s, out);
+  rocprim::inclusive_scan(tmp, tmp_bytes, rocprim::make_transform_iterator(in, WidenI32()), out + 1, (size_t)n,
+                          rocprim::plus<int64_t>(), s);
+  if (ck.flag) launch_cap_check(out + n, ck.cap, ck.flag, ck.bit, s);
+}
+void scan_paths(int64_t *z, int64_t *z_off, const CapCheck &ck_z, int64_t *cig, int64_t *cig_off, const CapCheck &ck_cig,
+                int64_t cap, const int64_t *n_dev, void *tmp, size_t tmp_bytes, hipStream_t s) {
+  if (cap <= kScanSmall) {
+    hipLaunchKernelGGL(k_scan_small2<ScanHead>, dim3(1), dim3(kScanThreads), 0, s, ScanHead{z, n_dev}, ScanHead{cig, n_dev},
+                       (int)cap, z_off, cig_off, ck_z, ck_cig);
+    return;
+  }
+  // sizes past the alignments count nothing in the scans over the capacity
+  launch_zero_tail(z, cap, n_dev, s);
+  launch_zero_tail(cig, cap, n_dev, s);
+  scan_i64(z, z_off, cap, tmp, tmp_bytes, s, ck_z);
+  scan_i64(cig, cig_off, cap, tmp, tmp_bytes, s, ck_cig);
+}
+void scan_cig_words(const Aln *alns, int64_t cap, const int64_t *n_dev, int32_t *words, int64_t *out, const CapCheck &ck,
+                    void *tmp, size_t tmp_bytes, hipStream_t s) {
+  if (cap <= kScanSmall) return scan_small(ScanWords{alns, n_dev}, cap, out, ck, s);
+  launch_cig_words(alns, cap, n_dev, words, s);
+  scan_i32(words, out, cap, tmp, tmp_bytes, s, ck);
+}
+// Before pass 1 of the slow reads: their pool offsets, and (once that pass is
+// through) where their intervals start; n_dev past cap sets `bit`.
+void scan_slow(int cap, const int32_t *n_dev, const int32_t *list, const int32_t *n_intv, int64_t *counts, int64_t *out,
+               const CapCheck &ck, int64_t base, int64_t *intv_base, int32_t bit, void *tmp, size_t tmp_bytes,
+               hipStream_t s) {
+  if (cap <= kScanSmall) {
+    hipLaunchKernelGGL(k_slow_offsets, dim3(1), dim3(kScanThreads), 0, s, ScanSlow{list, n_intv, n_dev}, cap, out, ck, base,
+                       intv_base, bit);
+    return;
+  }
+  launch_cap_check32(n_dev, cap, ck.flag, bit, s);
+  launch_gather_slow_counts(cap, n_dev, list, n_intv, counts, s);
+  scan_i64(counts, out, cap, tmp, tmp_bytes, s, ck);
+  launch_set_slow_base(cap, n_dev, list, out, base, intv_base, s);
 }
 
 // Counting sort of the lane tasks by descending key (kernels of its own:
