@@ -86,7 +86,31 @@ int main(int argc, char **argv) {
     if (tlen < 1) tlen = 1;
     if (tlen > qlen + 60) tlen = qlen + 60;
     if (tlen == qlen) ++tlen;
-    q.resize((size_t)qlen + 32, 0);
+    q.resize((size_t)qlen + 40, 0);
+    {
+      // the ungapped pass, 32 bases at a time, against one base at a time
+      Region g;
+      std::memset(&g, 0, sizeof g);
+      g.qe = qlen; g.rb = rb; g.re = rb + qlen; g.secondary = -1; g.score = qlen;
+      std::vector<uint8_t> qq(q.begin(), q.begin() + qlen);
+      qq.resize((size_t)qlen + 40, 0);
+      if (it % 3 == 0) o.mat[4] = o.mat[9] = o.mat[14] = o.mat[19] = -3;
+      if (it % 8 == 7) o.mat[7] = 2;  // no three-score matrix
+      uint32_t cig[16];
+      Aln a;
+      trace_and_finalize(x, o, qq.data(), qlen, g, 0, EhArray{nullptr, nullptr}, nullptr, cig, 0, a);
+      int nw = 0, nm = 0;
+      for (int i = 0; i < qlen; ++i) {
+        const int t = text_base(x, rb + i);
+        nw += o.mat[5 * t + qq[(size_t)i]];
+        nm += t != qq[(size_t)i];
+      }
+      if (a.nw_score != nw || a.nm != nm || a.n_core != 1) {
+        std::printf("FAIL ungapped %d: %d/%d %d/%d\n", it, a.nw_score, nw, a.nm, nm);
+        return 1;
+      }
+      if (it % 8 == 7) o.mat[7] = (int8_t)-o.b;
+    }
     // a band that the score's rule could give, or any above the lengths' difference
     Region g;
     std::memset(&g, 0, sizeof g);
