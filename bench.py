@@ -23,7 +23,7 @@ formatting; its SAM for that sample is compared byte for byte with `g3a mem
   python bench.py [--gpus 1] [--steps 3] [--warmup 1] [--config c4|c2|c3|c1]
                   [--form all|both|batched|plain|learned]
 
-Forms (identical output): plain (one wavefront per extension task), batched
+Forms (identical output): plain (16 lanes per extension task), batched
 (length-binned persistent lane engine) and learned (batched plus the
 learned-index seeding).  `value` is the learned form's rate when it ran (the
 metric's batched + learned form), else the batched form's; the others are
