@@ -820,8 +820,6 @@ constexpr int kRegionBigSlot32 = 88;  // k_region_large's
 // 0.20 ms, 27,801 tasks 1.33 against 0.46 ms, 281,296 tasks about 1.7 against
 // 2.9 ms.
 constexpr int32_t kExtGroupTasks = 1 << 16;
-// 568 tasks 0.20 ms either way; 11,517 sorted 0.35, unsorted 0.37 ms.
-constexpr int64_t kExtUnsorted = 1 << 12;
 
 static int64_t scale(double per, int64_t n, int64_t slack) { return (int64_t)(per * (double)n) + slack; }
 
@@ -929,11 +927,8 @@ static int run_extension(g3a_ctx *ctx, int64_t cap, const int64_t *n_dev, int64_
       ea.ctr = P<int32_t>(w.ext_ctr) + 4 * side;
       ea.rowbuf = plain ? nullptr : P<uint32_t>(w.ext_rowbuf);
       ea.cells = cells;
-      // few enough tasks for every group to start at once: their order is
-      // nothing to gain by, and sorting them takes four launches
-      if (group_ok && cap <= kExtUnsorted) ea.unsorted = sorted;
       launch_ext_classify(ea, s);
-      if (!ea.unsorted) ext_sort(ea.key, cap, n_dev, P<int32_t>(w.ext_hist), sorted, s);
+      ext_sort(ea.key, cap, n_dev, P<int32_t>(w.ext_hist), sorted, s);
       if (timed && !plain) HIPCK(hipEventRecord(ctx->kev[2 + 2 * side], s));
       if (group_ok) launch_ext_group(ea, ctx->n_cu, s);
       if (!plain && !(group_ok && cap <= kExtGroupTasks)) launch_ext_lane(ea, ctx->strip_rows, ctx->ext_packed, lane_blocks, s);

@@ -102,7 +102,6 @@ struct ExtSideArgs {
   const ExtRes *left;     // left results: h0 of the right side
   ExtRes *res;            // this side's results
   uint32_t *key;          // sort key: query length of lane tasks, 0 otherwise
-  int32_t *unsorted;      // lane task indices as classified, instead of keys (null: keys)
   const int32_t *sorted;  // lane task indices by descending key
   int32_t *slow_list;     // tasks for the one-wavefront kernel
   int32_t *ctr;           // [0] lane tasks [1] slow tasks [2] cursor over the lane tasks

@@ -1097,7 +1097,7 @@ __global__ void __launch_bounds__(256) k_ext_classify(ExtSideArgs a) {
   __syncthreads();
   const int64_t tile = (int64_t)blockIdx.x * (256 * kTilePer);
   const int64_t n = dcount(a.n_dev, a.n_tasks);
-  int n_lane = 0, slow_at[kTilePer], lane_at[kTilePer];
+  int n_lane = 0, slow_at[kTilePer];
 #pragma unroll
   for (int i = 0; i < kTilePer; ++i) {
     const int64_t t = tile + i * 256 + threadIdx.x;
@@ -1115,28 +1115,20 @@ __global__ void __launch_bounds__(256) k_ext_classify(ExtSideArgs a) {
       }
       if (lane) key = (uint32_t)st.qlen;
     }
-    if (a.unsorted) {
-      lane_at[i] = lane ? atomicAdd(&cnt[0], 1) : -1;
-    } else if (t < a.n_tasks) {
-      a.key[t] = key;
-    }
+    if (t < a.n_tasks) a.key[t] = key;
     n_lane += lane;
     slow_at[i] = slow ? atomicAdd(&cnt[1], 1) : -1;
   }
-  if (n_lane && !a.unsorted) atomicAdd(&cnt[0], n_lane);
+  if (n_lane) atomicAdd(&cnt[0], n_lane);
   __syncthreads();
   if (threadIdx.x == 0) {
-    base[0] = cnt[0] ? atomicAdd(a.ctr, cnt[0]) : 0;
+    if (cnt[0]) atomicAdd(a.ctr, cnt[0]);
     base[1] = cnt[1] ? atomicAdd(a.ctr + 1, cnt[1]) : 0;
   }
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < kTilePer; ++i)
     if (slow_at[i] >= 0) a.slow_list[base[1] + slow_at[i]] = (int32_t)(tile + i * 256 + threadIdx.x);
-  if (a.unsorted)
-#pragma unroll
-    for (int i = 0; i < kTilePer; ++i)
-      if (lane_at[i] >= 0) a.unsorted[base[0] + lane_at[i]] = (int32_t)(tile + i * 256 + threadIdx.x);
 }
 
 template <int R, bool SYM, bool PK>
