@@ -901,14 +901,12 @@ __device__ __forceinline__ int shr1(int src, int old) {
   return __builtin_amdgcn_update_dpp(old, src, 0x138 /* wave_shr:1 */, 0xf, 0xf, false);
 }
 
+// Over the 64 lanes, all active; the same scalar on each, so that what it
+// bounds is uniform to the compiler too
 __device__ __forceinline__ int wave_max_i32(int v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) {
-    int t = __shfl_xor(v, o);
-    v = v > t ? v : t;
-  }
-  return v;
+  return WaveLanes::get(WaveLanes::max_scan<64>(v, INT32_MIN, 0), 63);
 }
+__device__ __forceinline__ int wave_min_i32(int v) { return -wave_max_i32(-v); }
 __device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) {
@@ -1040,15 +1038,6 @@ __device__ ExtOut extend_wave(const Opt &o, int qlen, const uint8_t *qbuf, int t
 // the tasks that the 12-bit cells admit on the lane engine (g3a_ext.h) or on
 // 16 lanes each (g3a_ext_group.h), the rest on one wavefront each (extend_wave).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ int wave_min_i32(int v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) {
-    int t = __shfl_xor(v, o);
-    v = v < t ? v : t;
-  }
-  return v;
-}
-
 // Inputs of one side of task t (ExtendingPairGenerate, bwa/src/aux.cu:2101-2192;
 // localExtending, aux.cu:2289-2386): left = reversed read prefix against the
 // reversed reference before the seed, right = read suffix against the
@@ -1131,8 +1120,15 @@ __global__ void __launch_bounds__(256) k_ext_classify(ExtSideArgs a) {
     if (slow_at[i] >= 0) a.slow_list[base[1] + slow_at[i]] = (int32_t)(tile + i * 256 + threadIdx.x);
 }
 
+// What bounds it is packed VALU issue once the chip is full, the longest
+// tasks' columns before.  16-row strips fit four wavefronts a SIMD because the
+// wavefront's bounds are scalars (in registers of their own, and with the
+// lane addresses of their shuffles, they took 133 VGPRs and left three).  At
+// 16 blocks a compute unit 1,000,000 reads of 150 bases: 10.1 -> 9.5 ms; at 8
+// 11.7 -> 11.4 ms, and 250,000 reads 2.93 -> 3.00 ms (a column has 485
+// instructions, 475 with bounds in registers).
 template <int R, bool SYM, bool PK>
-__global__ void __launch_bounds__(64) k_ext_lane(ExtSideArgs a) {
+__global__ void __launch_bounds__(64, R == 16 ? 4 : 2) k_ext_lane(ExtSideArgs a) {
   if (a.stop && *a.stop) return;  // a capacity check before this kernel failed: the batch is redone
   constexpr int NW = R / 8;
   __shared__ uint32_t wt[6 * 64 * NW];
