@@ -87,7 +87,7 @@ EXPORTS = [
     "g3a_set_seed_blocks", "g3a_autotune_seed", "g3a_set_seed_order", "g3a_set_learned", "g3a_learned_stats",
     "g3a_last_intervals", "g3a_set_ext_packed", "g3a_ext_packed", "g3a_build_index_dev", "g3a_memcpy_text",
     "g3a_format_records", "g3a_copy_text", "g3a_bwa_align_noalloc", "g3a_set_wide_layout",
-    "g3a_mem_pestat", "g3a_mem_pair",
+    "g3a_mem_pestat", "g3a_mem_pair", "g3a_set_ext_group", "g3a_ext_engines",
 ]
 
 _lib = None
@@ -138,6 +138,8 @@ def load_library() -> C.CDLL:
     lib.g3a_mem_pestat.argtypes = [C.c_void_p, C.c_int, C.POINTER(PeStat)]
     lib.g3a_mem_pair.argtypes = [C.c_void_p, C.POINTER(PeStat), C.c_int64, C.c_void_p]
     lib.g3a_ext_packed.argtypes = [C.c_void_p]
+    lib.g3a_set_ext_group.argtypes = [C.c_void_p, C.c_int]
+    lib.g3a_ext_engines.argtypes = [C.c_void_p, C.POINTER(C.c_int)]
     lib.g3a_set_learned.argtypes = [C.c_void_p, C.c_int, C.POINTER(LearnedInfo)]
     lib.g3a_learned_stats.argtypes = [C.c_void_p, C.POINTER(C.c_int64)]
     lib.g3a_last_intervals.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.POINTER(C.c_int64)]
@@ -257,6 +259,16 @@ class Aligner:
     def set_ext_packed(self, packed: bool) -> None:
         """Lane engine with two strip rows per register (True) or one cell per lane."""
         self._check(self.lib.g3a_set_ext_packed(self.ctx, int(bool(packed))))
+
+    def set_ext_group(self, max_tasks: int) -> None:
+        """Most tasks a side of the batched form extends on 16 lanes each (0: none, the lane engine always)."""
+        self._check(self.lib.g3a_set_ext_group(self.ctx, max_tasks))
+
+    def ext_engines(self) -> tuple:
+        """What the left and right sides last ran on: 'lane', 'group', or None when there was no such task."""
+        v = (C.c_int * 2)()
+        self._check(self.lib.g3a_ext_engines(self.ctx, v))
+        return tuple((None, "lane", "group")[e] for e in v)
 
     def set_tuning(self, strip_rows: int, lane_blocks_per_cu: int, wave_blocks_per_cu: int) -> None:
         self._check(self.lib.g3a_set_tuning(self.ctx, strip_rows, lane_blocks_per_cu, wave_blocks_per_cu))

@@ -97,6 +97,14 @@ struct ScratchArena {
   size_t cap = 0, used = 0;
 };
 
+// Sides of at most this many tasks run on 16 lanes a task, larger ones on a
+// lane a task.  A lane's longest task takes 0.45 ms however few there are, and
+// a full chip of lanes 2.2 ns a task; 16 lanes take 0.1 ms and 5.5 ns a task.
+// Both sides of 150-base reads, lane against group: 568 tasks 1.28 against
+// 0.20 ms, 27,801 tasks 1.33 against 0.46 ms, 281,296 tasks about 1.7 against
+// 2.9 ms.
+constexpr int32_t kExtGroupTasks = 1 << 16;
+
 struct g3a_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -144,6 +152,7 @@ struct g3a_ctx {
   int n_cu = 0;
   int strip_rows = 16, lane_blocks_per_cu = 8, wave_blocks_per_cu = 8;
   int ext_packed = 1;  // lane engine: two strip rows per register in plain columns
+  int32_t ext_group_max = kExtGroupTasks;
   // host staging: readbacks, and page-locked copies of each batch's input
   // and output so that the transfers run at DMA speed
   int64_t *pinned = nullptr;
@@ -507,6 +516,7 @@ int g3a_device_alloc_sibling(g3a_ctx *src, int max_reads, int64_t max_bases, g3a
   ctx->lane_blocks_per_cu = src->lane_blocks_per_cu;
   ctx->wave_blocks_per_cu = src->wave_blocks_per_cu;
   ctx->ext_packed = src->ext_packed;
+  ctx->ext_group_max = src->ext_group_max;
   ctx->seed_blocks_per_cu = src->seed_blocks_per_cu;
   ctx->seed_block = src->seed_block;
   ctx->chain_serial = src->chain_serial;
@@ -813,14 +823,6 @@ constexpr int kNextReadSlot32 = 82;  // k_seed's read counter (int32)
 constexpr int kChainBigSlot32 = 84;   // k_chain_large's counts and cursors (4 int32)
 constexpr int kRegionBigSlot32 = 88;  // k_region_large's
 
-// Sides of at most this many tasks run on 16 lanes a task, larger ones on a
-// lane a task.  A lane's longest task takes 0.45 ms however few there are, and
-// a full chip of lanes 2.2 ns a task; 16 lanes take 0.1 ms and 5.5 ns a task.
-// Both sides of 150-base reads, lane against group: 568 tasks 1.28 against
-// 0.20 ms, 27,801 tasks 1.33 against 0.46 ms, 281,296 tasks about 1.7 against
-// 2.9 ms.
-constexpr int32_t kExtGroupTasks = 1 << 16;
-
 static int64_t scale(double per, int64_t n, int64_t slack) { return (int64_t)(per * (double)n) + slack; }
 
 static Caps plan_caps(const g3a_ctx *ctx, int n) {
@@ -912,7 +914,7 @@ static int run_extension(g3a_ctx *ctx, int64_t cap, const int64_t *n_dev, int64_
       ea.opt = ctx->opt;
       ea.side = side;
       ea.lane_opt_ok = plain ? group_ok : ext_lane_opt_ok(ctx->opt);
-      ea.group_max = !group_ok ? 0 : plain ? INT32_MAX : kExtGroupTasks;
+      ea.group_max = !group_ok ? 0 : plain ? INT32_MAX : ctx->ext_group_max;
       ea.n_tasks = cap;
       ea.n_dev = n_dev;
       ea.seq = P<uint8_t>(ctx->seq);
@@ -930,8 +932,8 @@ static int run_extension(g3a_ctx *ctx, int64_t cap, const int64_t *n_dev, int64_
       launch_ext_classify(ea, s);
       ext_sort(ea.key, cap, n_dev, P<int32_t>(w.ext_hist), sorted, s);
       if (timed && !plain) HIPCK(hipEventRecord(ctx->kev[2 + 2 * side], s));
-      if (group_ok) launch_ext_group(ea, ctx->n_cu, s);
-      if (!plain && !(group_ok && cap <= kExtGroupTasks)) launch_ext_lane(ea, ctx->strip_rows, ctx->ext_packed, lane_blocks, s);
+      if (ea.group_max > 0) launch_ext_group(ea, ctx->n_cu, s);
+      if (!plain && cap > ea.group_max) launch_ext_lane(ea, ctx->strip_rows, ctx->ext_packed, lane_blocks, s);
       if (timed && !plain) HIPCK(hipEventRecord(ctx->kev[3 + 2 * side], s));
       launch_ext_wave(ea, wave_blocks, s);
       if (timed && !plain) {
@@ -1140,7 +1142,7 @@ static std::string graph_key(const g3a_ctx *ctx, int n, const Caps &c) {
   put(&ctx->idx, sizeof ctx->idx);
   put(&ctx->opt, sizeof ctx->opt);
   const int v[] = {ctx->form, ctx->strip_rows, ctx->lane_blocks_per_cu, ctx->wave_blocks_per_cu, ctx->ext_packed,
-                   ctx->seed_blocks_per_cu, ctx->seed_block, ctx->run_tb_threads, ctx->run_lane_blocks,
+                   ctx->ext_group_max, ctx->seed_blocks_per_cu, ctx->seed_block, ctx->run_tb_threads, ctx->run_lane_blocks,
                    ctx->run_slow_chunk, ctx->chain_serial};
   put(v, sizeof v);
   put(&ctx->buf_gen, sizeof ctx->buf_gen);
@@ -1554,8 +1556,20 @@ int g3a_autotune(g3a_ctx *ctx, int *strip_rows, int *lane_blocks_per_cu, float *
   if (!ctx->has_output || ctx->w != &ctx->own)
     return fail(ctx, G3A_E_STATE, "autotune needs a batch aligned on the device by g3a_bwa_align");
   HIPCK(hipSetDevice(ctx->device));
-  const int form = ctx->form, sr0 = ctx->strip_rows, lb0 = ctx->lane_blocks_per_cu, pk0 = ctx->ext_packed;
+  const int sr0 = ctx->strip_rows, lb0 = ctx->lane_blocks_per_cu, pk0 = ctx->ext_packed;
+  struct Restore {
+    g3a_ctx *c;
+    int form;
+    int32_t group_max;
+    ~Restore() {
+      c->form = form;
+      c->ext_group_max = group_max;
+    }
+  } restore{ctx, ctx->form, ctx->ext_group_max};
+  // the settings are the lane engine's: it is what is timed, also for a batch
+  // small enough for 16 lanes a task
   ctx->form = G3A_FORM_BATCHED;
+  ctx->ext_group_max = 0;
   int64_t *cells = P<int64_t>(ctx->w->counters) + 24;
   // the last batch's tasks: their capacity and their count on the device
   const int64_t cap = ctx->caps.tasks, *n_dev = P<int64_t>(ctx->w->task_off) + ctx->n_reads;
@@ -1595,7 +1609,6 @@ int g3a_autotune(g3a_ctx *ctx, int *strip_rows, int *lane_blocks_per_cu, float *
   if (int rc = run_extension(ctx, cap, n_dev, cells, false)) return rc;
   HIPCK(hipMemcpyAsync(cells, &saved, 8, hipMemcpyHostToDevice, ctx->stream));
   HIPCK(hipStreamSynchronize(ctx->stream));
-  ctx->form = form;
   if (strip_rows) *strip_rows = bsr;
   if (lane_blocks_per_cu) *lane_blocks_per_cu = blb;
   if (best_ms) *best_ms = best;
@@ -1858,6 +1871,27 @@ int g3a_set_ext_packed(g3a_ctx *ctx, int packed) {
 }
 
 int g3a_ext_packed(const g3a_ctx *ctx) { return ctx ? ctx->ext_packed : -1; }
+
+static_assert(kEngineNone == G3A_ENGINE_NONE && kEngineLane == G3A_ENGINE_LANE && kEngineGroup == G3A_ENGINE_GROUP,
+              "the ABI's numbers");
+int g3a_set_ext_group(g3a_ctx *ctx, int max_tasks) {
+  if (!ctx || max_tasks < 0) return G3A_E_ARG;
+  ctx->ext_group_max = max_tasks;
+  return G3A_OK;
+}
+
+int g3a_ext_engines(g3a_ctx *ctx, int engines[2]) {
+  if (!ctx || !engines) return G3A_E_ARG;
+  if (!ctx->has_output || ctx->w != &ctx->own)
+    return fail(ctx, G3A_E_STATE, "the engines are those of a batch aligned by g3a_bwa_align");
+  engines[0] = engines[1] = G3A_ENGINE_NONE;
+  if (!ctx->n_reads) return G3A_OK;
+  HIPCK(hipSetDevice(ctx->device));
+  int32_t ctr[8];
+  HIPCK(hipMemcpy(ctr, ctx->w->ext_ctr.p, sizeof ctr, hipMemcpyDeviceToHost));
+  for (int side = 0; side < 2; ++side) engines[side] = ctr[4 * side + 3];
+  return G3A_OK;
+}
 
 int g3a_last_stats(const g3a_ctx *ctx, float ms[6], int64_t work[6]) {
   if (!ctx || !ms || !work) return G3A_E_ARG;

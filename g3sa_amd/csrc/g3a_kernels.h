@@ -79,6 +79,8 @@ struct CompactArgs {
   Task *tasks;
 };
 
+enum : int32_t { kEngineNone, kEngineLane, kEngineGroup };  // what a side's lane tasks ran on
+
 // Result of one side of one extension task.
 struct ExtRes {
   int32_t score, qle, tle, pad;
@@ -104,7 +106,7 @@ struct ExtSideArgs {
   uint32_t *key;          // sort key: query length of lane tasks, 0 otherwise
   const int32_t *sorted;  // lane task indices by descending key
   int32_t *slow_list;     // tasks for the one-wavefront kernel
-  int32_t *ctr;           // [0] lane tasks [1] slow tasks [2] cursor over the lane tasks
+  int32_t *ctr;           // [0] lane tasks [1] slow tasks [2] cursor over the lane tasks [3] the engine they ran on
   int32_t group_max;      // up to this many lane tasks run on 16 lanes each
   uint32_t *rowbuf;       // kExtQCap * 64 words per lane-kernel block
   int64_t *cells;

@@ -1136,6 +1136,7 @@ __global__ void __launch_bounds__(64, R == 16 ? 4 : 2) k_ext_lane(ExtSideArgs a)
   uint32_t *rb = a.rowbuf + (size_t)blockIdx.x * (kExtQCap * 64) + lane;
   const int n_lane = a.ctr[0];
   if (n_lane <= a.group_max) return;  // k_ext_group's
+  if (blockIdx.x == 0 && lane == 0) a.ctr[3] = kEngineLane;
   int64_t cells = 0;
   for (;;) {
     int chunk = 0;
@@ -1195,6 +1196,7 @@ __global__ void __launch_bounds__(64, 3) k_ext_group(ExtSideArgs a) {
   if (n_lane > a.group_max) return;  // k_ext_lane's
   __shared__ ExtGroupStage stage[4];
   const int lane = threadIdx.x, gl = lane & 15, gb = lane & 48;
+  if (blockIdx.x == 0 && lane == 0 && n_lane) a.ctr[3] = kEngineGroup;
   int64_t cells = 0;
   for (;;) {
     WaveLanes::lds_sync();  // the wavefront meets here, as in k_chain_large

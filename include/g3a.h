@@ -248,13 +248,24 @@ int g3a_set_ext_packed(g3a_ctx *ctx, int packed);
  * small enough to check.  No reference counterpart. */
 int g3a_set_wide_layout(g3a_ctx *ctx, int on);
 int g3a_ext_packed(const g3a_ctx *ctx);
+/* Batched form: sides of at most max_tasks tasks run on 16 lanes a task, larger
+ * ones on the lane engine (0: always; default 65536).  Identical results.  No
+ * reference counterpart. */
+int g3a_set_ext_group(g3a_ctx *ctx, int max_tasks);
+/* The engine that the left [0] and right [1] sides last ran on: of the batch
+ * last aligned, or of g3a_autotune's last setting.  Tasks outside the 16-bit
+ * engines' domain are not counted.  No reference counterpart. */
+#define G3A_ENGINE_NONE 0  /* no such task */
+#define G3A_ENGINE_LANE 1  /* a lane per task */
+#define G3A_ENGINE_GROUP 2 /* 16 lanes per task */
+int g3a_ext_engines(g3a_ctx *ctx, int engines[2]);
 /* Autotuner of the batched form: on the batch last aligned (its tasks are
- * still on the device), time the extension stage for each lane arithmetic
- * (packed or not), strip height (16, 32) and persistent lane blocks per
- * compute unit (2, 4, 8, 16), keep the fastest setting on the context and
- * report it (the arithmetic through g3a_ext_packed).  Results are identical
- * for every setting; the batch's output is left as it was.  No reference
- * counterpart. */
+ * still on the device), time the extension stage on the lane engine, whatever
+ * the batch's size, for each arithmetic of it (packed or not), strip height
+ * (16, 32) and persistent lane blocks per compute unit (2, 4, 8, 16), keep the
+ * fastest setting on the context and report it (the arithmetic through
+ * g3a_ext_packed).  Results are identical for every setting; the batch's
+ * output is left as it was.  No reference counterpart. */
 int g3a_autotune(g3a_ctx *ctx, int *strip_rows, int *lane_blocks_per_cu, float *best_ms);
 /* Persistent seeding blocks per compute unit at the current block size
  * (g3a_set_seed_grid); 0: the occupancy maximum.  No reference counterpart. */
