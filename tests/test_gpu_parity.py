@@ -41,14 +41,34 @@ def compare(gpu: g3sa_amd.Result, ref: dict, label: str) -> None:
 
 
 # (form, tuning, seed order, seeding grid (threads per block, blocks per
-# CU), packed lane arithmetic): the plain form and the batched form at both
-# strip heights with two strip rows per register, and at 16 rows with one
-# cell per lane; reads seeded in minimizer order and in input order; seeding
-# grids of 1024, 512, 256 and 128 threads per block, whose LDS shares hold
-# different numbers of LEP entries per thread (the rest of a list spills to
-# its global slice)
-VARIANTS = [("plain", None, 1, (1024, 1), 1), ("batched", (16, 8, 8), 1, (128, 10), 1),
-            ("batched", (32, 4, 8), 0, (256, 4), 1), ("batched", (16, 8, 8), 0, (512, 0), 0)]
+# CU), packed lane arithmetic, most tasks a side extends on 16 lanes each): the
+# plain form; the batched form on the lane engine (no side on 16 lanes) at both
+# strip heights with two strip rows per register, and at 16 rows with one cell
+# per lane; and on the engine that it picks for a batch of this size.  Reads
+# are seeded in minimizer order and in input order, by grids of 1024, 512, 256
+# and 128 threads per block.
+VARIANTS = [("plain", None, 1, (1024, 1), 1, 0), ("batched", (16, 8, 8), 1, (128, 10), 1, 0),
+            ("batched", (32, 4, 8), 0, (256, 4), 1, 0), ("batched", (16, 8, 8), 0, (512, 0), 0, 0),
+            ("batched", (16, 8, 8), 1, (1024, 1), 1, 65536)]
+
+
+def set_variant(al, variant) -> None:
+    form, tuning, ordered, blocks, packed, group = variant
+    al.set_form(form)
+    if tuning:
+        al.set_tuning(*tuning)
+    al.set_seed_order(ordered)
+    al.set_seed_grid(*blocks)
+    al.set_ext_packed(packed)
+    al.set_ext_group(group)
+
+
+def check_engines(al, variant) -> int:
+    """Each side ran on the variant's engine; the number of sides with tasks for it."""
+    want = "group" if variant[0] == "plain" or variant[5] else "lane"
+    ran = [e for e in al.ext_engines() if e]
+    assert all(e == want for e in ran), f"{variant}: sides ran on {ran}"
+    return len(ran)
 
 
 def run_both(ds, oracle, seq, off, label, max_reads=None, wide=False, variants=None):
@@ -60,17 +80,12 @@ def run_both(ds, oracle, seq, off, label, max_reads=None, wide=False, variants=N
         oracle.lib.orc_index_free(idx)
     with g3sa_amd.Aligner(str(ds.prefix), max_reads=max(max_reads or n, 1),
                           max_bases=max(int(off[-1]), 1), wide_layout=wide) as al:
-        for form, tuning, ordered, blocks, packed in variants or VARIANTS:
-            print(f"[parity] {label}: {n} reads, form {form} {tuning} seed order {ordered} blocks {blocks} "
-                  f"packed {packed}", flush=True)
-            al.set_form(form)
-            if tuning:
-                al.set_tuning(*tuning)
-            al.set_seed_order(ordered)
-            al.set_seed_grid(*blocks)
-            al.set_ext_packed(packed)
+        for v in variants or VARIANTS:
+            print(f"[parity] {label}: {n} reads, (form, tuning, seed order, blocks, packed, group) {v}", flush=True)
+            set_variant(al, v)
             got = al.align(seq, off)
-            compare(got, ref, f"{label} [{form} {tuning} order {ordered}]")
+            compare(got, ref, f"{label} {v}")
+            check_engines(al, v)
             # seeds resolved by the GPU equal the oracle's SA lookups
             assert got.work["n_seeds"] == ref["work"]["sa_reads"], label
     return got, ref
@@ -133,14 +148,17 @@ def test_single_read_and_repeated_batches(ds_c1, oracle):
         oracle.lib.orc_index_free(idx)
 
 
-def _with_scoring(oracle, w=None, b=None):
-    """Matching option blocks for the oracle and the library."""
+def _with_scoring(oracle, w=None, b=None, ins=None):
+    """Matching option blocks for the oracle and the library; ins: costs of
+    opening and extending an insertion."""
     oo = type(oracle.opt)()
     C.pointer(oo)[0] = oracle.opt
     go = g3sa_amd.default_opt()
     for o in (oo, go):
         if w is not None:
             o.w = w
+        if ins is not None:
+            o.o_ins, o.e_ins = ins
         if b is not None:
             o.b = b
             for i in range(4):
@@ -149,30 +167,26 @@ def _with_scoring(oracle, w=None, b=None):
     return oo, go
 
 
-@pytest.mark.parametrize("w,b", [(20, None), (None, 9)])
-def test_scoring_variants_parity(ds_c1, oracle, w, b):
+@pytest.mark.parametrize("w,b,ins", [(20, None, None), (None, 9, None), (None, None, (4, 2)), (20, None, (4, 2))])
+def test_scoring_variants_parity(ds_c1, oracle, w, b, ins):
     """A narrow band (the column limit, corner rule and quirk rows of the
     reference's cell set apply to many cells of the lane engine's general
-    columns) and a mismatch score outside the lane engine's 4-bit range
-    (every task takes the one-wavefront kernel)."""
+    columns), a mismatch score outside the lane engine's 4-bit range (every
+    task takes the one-wavefront kernel) and insertions that cost other than
+    deletions."""
     names, seq, off, _ = g3sa_amd.read_fastq(str(ds_c1.reads["c3"]), limit=1500)
-    oo, go = _with_scoring(oracle, w, b)
+    oo, go = _with_scoring(oracle, w, b, ins)
     idx = oracle.load(ds_c1.prefix)
     try:
         ref = oracle.align(idx, seq, off, threads=oracle_threads(), opt=oo)
     finally:
         oracle.lib.orc_index_free(idx)
     with g3sa_amd.Aligner(str(ds_c1.prefix), max_reads=len(off) - 1, max_bases=int(off[-1]), opt=go) as al:
-        for form, tuning, ordered, blocks, packed in VARIANTS:
-            print(f"[parity] scoring w={w} b={b}: form {form} {tuning} seed order {ordered} blocks {blocks} "
-                  f"packed {packed}", flush=True)
-            al.set_form(form)
-            if tuning:
-                al.set_tuning(*tuning)
-            al.set_seed_order(ordered)
-            al.set_seed_grid(*blocks)
-            al.set_ext_packed(packed)
-            compare(al.align(seq, off), ref, f"scoring w={w} b={b} [{form} {tuning} order {ordered}]")
+        for v in VARIANTS:
+            print(f"[parity] scoring w={w} b={b} ins={ins}: {v}", flush=True)
+            set_variant(al, v)
+            compare(al.align(seq, off), ref, f"scoring w={w} b={b} ins={ins} {v}")
+            assert check_engines(al, v) == (0 if b else 2)
 
 
 def test_empty_batch(ds_c1):
