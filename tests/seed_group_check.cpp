@@ -5,7 +5,9 @@
 //   seed_group_check PREFIX READS [MIN_SEED_LEN]
 // Groups of 16 lanes with 64 entries (the fast path, which may give a read
 // up) and of 64 lanes with 320 (which may not), in the narrow and the wide
-// layout and with the full suffix array.  Prints "ok key=value ..." or the first failure.
+// layout and with the full suffix array.  Prints "ok key=value ..." or the
+// first failure; given_up_* and compared_* are the reads given up and the
+// intervals compared of the 16-lane groups, by form.
 #include "g3sa_amd/csrc/g3a_dev.h"
 #include "g3sa_amd/csrc/g3a_index.h"
 #include "g3sa_amd/csrc/g3a_layout.h"
@@ -136,7 +138,7 @@ int main(int argc, char **argv) {
 
   std::mt19937_64 rng(99);
   Fibers fb;
-  int64_t n_iv = 0, given_up = 0, st1 = 0, st16 = 0, st64 = 0, stw = 0, stl = 0;
+  int64_t n_iv = 0, given_up[3] = {0, 0, 0}, compared[3] = {0, 0, 0}, st1 = 0, st16 = 0, st64 = 0, stw = 0, stl = 0;
   for (int i = 0; i < n_reads; ++i) {
     // all lengths up to the limit, short ones and the limit more often
     int len = i % 7 == 0 ? (int)(rng() % 45) : i % 7 == 1 ? kMaxReadLen - (int)(rng() % 3) : 36 + (int)(rng() % 285);
@@ -183,7 +185,7 @@ int main(int argc, char **argv) {
                             : group_read<64, 5, uint32_t, true>(fb, xl, o, buf, off, len, 4096, got, ns, stl);
       if (!ok) {
         if (form & 1) return fail("wavefront group gave up", i, len, form);
-        ++given_up;
+        ++given_up[form / 2];
         continue;
       }
       if (got.size() != ref.size()) return fail("intervals", i, form, (long long)got.size() - (long long)ref.size());
@@ -192,10 +194,14 @@ int main(int argc, char **argv) {
         const Intv &u = ref[k], &v = got[k];
         if (u.k != v.k || u.s != v.s || u.m != v.m || u.n != v.n) return fail("interval", i, form, (long long)k);
       }
+      if (!(form & 1)) compared[form / 2] += (int64_t)ref.size();
     }
   }
-  std::printf("ok reads=%d intervals=%lld given_up=%lld steps_thread=%lld steps_16=%lld steps_64=%lld steps_wide=%lld steps_text=%lld\n",
-              n_reads, (long long)n_iv, (long long)given_up, (long long)st1, (long long)st16, (long long)st64,
-              (long long)stw, (long long)stl);
+  std::printf("ok reads=%d intervals=%lld", n_reads, (long long)n_iv);
+  const char *name[3] = {"narrow", "wide", "text"};
+  for (int f = 0; f < 3; ++f)
+    std::printf(" given_up_%s=%lld compared_%s=%lld", name[f], (long long)given_up[f], name[f], (long long)compared[f]);
+  std::printf(" steps_thread=%lld steps_16=%lld steps_64=%lld steps_wide=%lld steps_text=%lld\n", (long long)st1,
+              (long long)st16, (long long)st64, (long long)stw, (long long)stl);
   return 0;
 }

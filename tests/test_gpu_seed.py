@@ -58,3 +58,17 @@ def test_seeding_edges(ds_rep, oracle, form, min_seed_len):
         print(f"[seed] {form}, min_seed_len {min_seed_len}: {n} reads", flush=True)
         al.align(seq, off)
         _intervals_equal((counts, flat), al.intervals(), f"{form} min_seed_len {min_seed_len}")
+
+
+@pytest.mark.parametrize("form", ["narrow", "wide", "learned"])
+def test_ordinary_reads_stay_on_16_lanes(ds_c1, form):
+    """A group that gives up leaves its read to the slow path, whose output is
+    the same: reads of 150 bases at 1% substitutions on a text without repeats
+    have short lists and few matches, so hardly any may go there."""
+    _, seq, off, _ = g3sa_amd.read_fastq(str(ds_c1.reads["main"]))
+    n = len(off) - 1
+    with g3sa_amd.Aligner(str(ds_c1.prefix), max_reads=n, max_bases=int(off[-1]), wide_layout=form == "wide") as al:
+        if form == "learned":
+            al.set_learned(1)
+        got = al.align(seq, off)
+    assert got.work["n_slow_reads"] <= n // 100

@@ -38,4 +38,13 @@ def test_seed_group_equals_one_thread(checker, repeats, min_seed_len):
                        timeout=600)
     assert r.returncode == 0 and r.stdout.startswith("ok"), r.stdout + r.stderr
     s = {k: float(v) for k, v in (t.split("=") for t in r.stdout.split()[1:])}
-    assert s["intervals"] > 0 and s["given_up"] < 6 * 300
+    # With seeds longer than the table's 12 bases a 16-lane group gives up the
+    # reads of one repeated word (one in 29) and some of the text's tandem
+    # repeats (3% of it): a tenth at most.  Shorter seeds are many more and may
+    # fill the 64 output slots of a long read, but not of the shorter half.
+    # A third of the 233 text reads of 36 bases or more have no errors, so each
+    # of those that is not given up has an interval.
+    most = 30 if min_seed_len > 12 else 150
+    for form in ("narrow", "wide", "text"):
+        assert s[f"given_up_{form}"] <= most, form
+        assert s[f"compared_{form}"] >= 300 * 6 // 7 * 10 // 11 // 3 - 30, form
