@@ -62,8 +62,8 @@ struct Work {
   DevBuf aln_reg, aln_read, aln_rank, z_size, cig_size, z_off, cig_off, z, cigar, alns;
   DevBuf cig_words, cig_coff, cig_out;  // compacted CIGARs for the host copy
   DevBuf scan_tmp, totals;
-  // batched-form extension
-  DevBuf ext_res[2], ext_key, ext_sorted, ext_slow, ext_ctr, ext_hist, ext_rowbuf;
+  // extension
+  DevBuf ext_ctr, ext_hist, ext_rowbuf;
 };
 
 // Capacities of one attempt at a batch: the buffers the pipeline writes are
@@ -849,20 +849,23 @@ static void free_graph(g3a_ctx *ctx) {
 
 namespace {
 
-// Per-task arrays of the extension stage.  The seed sort's copy and the chains
-// are dead by then, and a batch has no more tasks than seeds: the arrays lie in
-// those buffers unless the capacities grew apart.
-bool ext_shares(const Work &w, int64_t cap) {
-  return w.seeds2.bytes >= (size_t)cap * 2 * sizeof(ExtRes) && w.ch.bytes >= (size_t)cap * 12;
+// Per-task arrays of the extension stage, for `cap` tasks: a batch's capacity
+// for tasks is at most that for seeds, and the seed sort's copy, the reads' own
+// task lists and the chains are dead by then, so the arrays lie in those.
+struct ExtArrays {
+  ExtRes *res[2];
+  uint32_t *key;
+  int32_t *sorted, *slow;
+};
+static_assert(sizeof(Seed) >= sizeof(ExtRes) && sizeof(Task) >= sizeof(ExtRes) && sizeof(ChainTmp) >= 3 * 4,
+              "a seed's share of the buffers holds a task's arrays");
+ExtArrays ext_arrays(Work &w, int64_t cap) {
+  int32_t *v = P<int32_t>(w.ch);
+  return ExtArrays{{P<ExtRes>(w.seeds2), P<ExtRes>(w.tasks_tmp)}, (uint32_t *)v, v + cap, v + 2 * cap};
 }
-// Buffers of the extension stage for `cap` tasks.
-int alloc_ext(g3a_ctx *ctx, int64_t cap) {
+// The extension stage's other buffers.
+int alloc_ext(g3a_ctx *ctx) {
   Work &w = *ctx->w;
-  if (!ext_shares(w, cap) &&
-      (ensure(ctx, w.ext_res[0], (size_t)cap * sizeof(ExtRes)) || ensure(ctx, w.ext_res[1], (size_t)cap * sizeof(ExtRes)) ||
-       ensure(ctx, w.ext_key, (size_t)cap * 4) || ensure(ctx, w.ext_sorted, (size_t)cap * 4) ||
-       ensure(ctx, w.ext_slow, (size_t)cap * 4)))
-    return G3A_E_HIP;
   const int lane_blocks = ctx->arena ? ctx->run_lane_blocks : ctx->n_cu * ctx->lane_blocks_per_cu;
   return ensure(ctx, w.ext_ctr, 2 * 4 * sizeof(int32_t)) || ensure(ctx, w.ext_hist, 1024 * 4) ||
          (ctx->form != G3A_FORM_PLAIN && ensure(ctx, w.ext_rowbuf, (size_t)lane_blocks * kExtQCap * 64 * 4));
@@ -884,7 +887,7 @@ int alloc_batch(g3a_ctx *ctx, int n, const Caps &c) {
       alloc_paths(ctx, c.z, c.cig) || ensure(ctx, w.cig_words, (size_t)c.alns * 4 + 4) ||
       ensure(ctx, w.cig_coff, (size_t)(c.alns + 1) * 8) || ensure(ctx, w.cig_out, (size_t)c.used * 4 + 64))
     return alloc_fail(ctx);
-  if (alloc_ext(ctx, c.tasks)) return alloc_fail(ctx);
+  if (alloc_ext(ctx)) return alloc_fail(ctx);
   return 0;
 }
 
@@ -902,9 +905,7 @@ static int run_extension(g3a_ctx *ctx, int64_t cap, const int64_t *n_dev, int64_
     const int lane_blocks = ctx->arena ? ctx->run_lane_blocks : ctx->n_cu * ctx->lane_blocks_per_cu,
               wave_blocks = ctx->n_cu * ctx->wave_blocks_per_cu;
     const bool group_ok = ext_group_opt_ok(ctx->opt);
-    const bool shared = ext_shares(w, cap);
-    ExtRes *res[2] = {shared ? P<ExtRes>(w.seeds2) : P<ExtRes>(w.ext_res[0]),
-                      shared ? P<ExtRes>(w.seeds2) + cap : P<ExtRes>(w.ext_res[1])};
+    const ExtArrays v = ext_arrays(w, cap);
     launch_fill_i32(P<int32_t>(w.ext_ctr), 8, 0, s);
     if (timed && plain) HIPCK(hipEventRecord(ctx->kev[3], s));
     for (int side = 0; side < 2; ++side) {
@@ -920,17 +921,16 @@ static int run_extension(g3a_ctx *ctx, int64_t cap, const int64_t *n_dev, int64_
       ea.seq = P<uint8_t>(ctx->seq);
       ea.off = P<int32_t>(ctx->off);
       ea.tasks = P<Task>(w.tasks);
-      ea.left = res[0];
-      ea.res = res[side];
-      ea.key = shared ? P<uint32_t>(w.ch) : P<uint32_t>(w.ext_key);
-      int32_t *sorted = shared ? P<int32_t>(w.ch) + cap : P<int32_t>(w.ext_sorted);
-      ea.sorted = sorted;
-      ea.slow_list = shared ? P<int32_t>(w.ch) + 2 * cap : P<int32_t>(w.ext_slow);
+      ea.left = v.res[0];
+      ea.res = v.res[side];
+      ea.key = v.key;
+      ea.sorted = v.sorted;
+      ea.slow_list = v.slow;
       ea.ctr = P<int32_t>(w.ext_ctr) + 4 * side;
       ea.rowbuf = plain ? nullptr : P<uint32_t>(w.ext_rowbuf);
       ea.cells = cells;
       launch_ext_classify(ea, s);
-      ext_sort(ea.key, cap, n_dev, P<int32_t>(w.ext_hist), sorted, s);
+      ext_sort(v.key, cap, n_dev, P<int32_t>(w.ext_hist), v.sorted, s);
       if (timed && !plain) HIPCK(hipEventRecord(ctx->kev[2 + 2 * side], s));
       if (ea.group_max > 0) launch_ext_group(ea, ctx->n_cu, s);
       if (!plain && cap > ea.group_max) launch_ext_lane(ea, ctx->strip_rows, ctx->ext_packed, lane_blocks, s);
@@ -950,8 +950,8 @@ static int run_extension(g3a_ctx *ctx, int64_t cap, const int64_t *n_dev, int64_
     fa.n_tasks = cap;
     fa.n_dev = n_dev;
     fa.tasks = P<Task>(ctx->w->tasks);
-    fa.left = res[0];
-    fa.right = res[1];
+    fa.left = v.res[0];
+    fa.right = v.res[1];
     fa.regs = P<Region>(ctx->w->regs);
     launch_ext_finish(fa, s);
   }
@@ -1159,8 +1159,10 @@ static int align_batch(g3a_ctx *ctx) {
   ctx->has_output = false;
   ctx->total_seeds = ctx->total_tasks = ctx->total_alns = ctx->total_cig = ctx->n_slow = 0;
   Caps c = plan_caps(ctx, n);
+  int64_t tasks = c.tasks;
   for (int attempt = 0;; ++attempt) {
     if (attempt == 8) return fail(ctx, G3A_E_INTERNAL, "batch capacities did not settle");
+    c.tasks = std::min(tasks, c.seeds);  // a task is a seed of its own
     if (ctx->arena) {  // an allocation-free attempt carves the scratch afresh
       ctx->arena->used = 0;
       ctx->scratch_work = Work{};
@@ -1208,7 +1210,7 @@ static int align_batch(g3a_ctx *ctx) {
       if (flags & kOvSlow) c.slow = (int)std::min<int64_t>(n, grow(c.slow, n_slow));
       else if (flags & kOvPool) c.pool = grow(c.pool, t[kTotPool]);
       else if (flags & kOvSeeds) c.seeds = grow(c.seeds, t[kTotSeeds]);
-      else if (flags & kOvTasks) c.tasks = grow(c.tasks, t[kTotTasks]);
+      else if (flags & kOvTasks) tasks = grow(c.tasks, t[kTotTasks]);
       else if (flags & kOvAlns) c.alns = grow(c.alns, t[kTotAlns]);
       else {
         if (flags & kOvZ) c.z = grow(c.z, t[kTotZ]);
@@ -1588,7 +1590,7 @@ int g3a_autotune(g3a_ctx *ctx, int *strip_rows, int *lane_blocks_per_cu, float *
       // first run warms the buffers of this shape, the second is timed
       for (int rep = 0; rep < 2; ++rep) {
         HIPCK(hipEventRecord(ctx->ev[6], ctx->stream));
-        if (alloc_ext(ctx, cap)) return G3A_E_HIP;
+        if (alloc_ext(ctx)) return G3A_E_HIP;
         if (int rc = run_extension(ctx, cap, n_dev, cells, false)) return rc;
         HIPCK(hipEventRecord(ctx->ev[7], ctx->stream));
         HIPCK(hipEventSynchronize(ctx->ev[7]));
@@ -1605,7 +1607,7 @@ int g3a_autotune(g3a_ctx *ctx, int *strip_rows, int *lane_blocks_per_cu, float *
   ctx->lane_blocks_per_cu = blb;
   ctx->ext_packed = bpk;
   // leave the regions and counters as the aligned batch had them
-  if (alloc_ext(ctx, cap)) return G3A_E_HIP;
+  if (alloc_ext(ctx)) return G3A_E_HIP;
   if (int rc = run_extension(ctx, cap, n_dev, cells, false)) return rc;
   HIPCK(hipMemcpyAsync(cells, &saved, 8, hipMemcpyHostToDevice, ctx->stream));
   HIPCK(hipStreamSynchronize(ctx->stream));
@@ -1931,8 +1933,7 @@ void g3a_destroy(g3a_ctx *ctx) {
                     &ctx->own.cig_size, &ctx->own.z_off, &ctx->own.cig_off, &ctx->own.z, &ctx->own.cigar, &ctx->own.alns, &ctx->own.scan_tmp,
                     &ctx->own.cig_words, &ctx->own.cig_coff, &ctx->own.cig_out, &ctx->own.seed_key, &ctx->own.seed_key2, &ctx->own.seed_idx,
                     &ctx->own.seed_order, &ctx->own.seed_sort_tmp,
-                    &ctx->own.ext_res[0], &ctx->own.ext_res[1], &ctx->own.ext_key, &ctx->own.ext_hist, &ctx->own.totals,
-                    &ctx->own.ext_sorted, &ctx->own.ext_slow, &ctx->own.ext_ctr, &ctx->own.ext_rowbuf,
+                    &ctx->own.ext_hist, &ctx->own.totals, &ctx->own.ext_ctr, &ctx->own.ext_rowbuf,
                     &ctx->own.eh_pool, &ctx->own.tb_order, &ctx->own.tb_ctr, &ctx->li_saf, &ctx->li_keys,
                     &ctx->li_root, &ctx->li_leaf, &ctx->li_knot, &ctx->li_leaf_a, &ctx->li_short, &ctx->li_ctr,
                     &ctx->ctg_names, &ctx->ctg_name_off, &ctx->log_tab, &ctx->names, &ctx->name_off, &ctx->quals,

@@ -66,3 +66,20 @@ def test_noalloc_refuses_batches_over_its_limit(ds_c1):
         al.upload(seq[:off[100]], off[:101])
         al.run_noalloc()
         assert al.download().n_alns > 90
+
+
+@pytest.mark.parametrize("form,per_read", [("plain", 1000), ("batched", 820)])
+def test_noalloc_takes_as_many_tasks_as_seeds(ds_c1, form, per_read):
+    """Repeats can give nearly as many extension tasks as seeds: 1000 reads of
+    150 bases with room for per_read of each fit the scratch array (265 bytes a
+    seed and its task; per-task arrays of the extension beside them would not
+    fit)."""
+    _, seq, off, _ = g3sa_amd.read_fastq(str(ds_c1.reads["main"]), limit=1000)
+    with g3sa_amd.Aligner(str(ds_c1.prefix), max_reads=1000, max_bases=int(off[-1])) as al:
+        al.set_form(form)
+        al.upload(seq, off)
+        al.run()
+        ref = al.download()
+        al.set_batch_caps(per_read, per_read, 1, 8, 4, 4, 64)
+        al.run_noalloc()
+        _same(al.download(), ref, form)
