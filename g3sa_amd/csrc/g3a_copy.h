@@ -16,8 +16,8 @@
 #include <cstddef>
 #include <cstdint>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -43,7 +43,7 @@ class CopyCrew {
     if (threads_.empty() && !failed_) {
       try {
         for (int i = 0; i < kHelpers; ++i) threads_.emplace_back([this] { help(); });
-      } catch (const std::system_error &) {
+      } catch (const std::exception &) {  // no thread, or no memory for one
         failed_ = threads_.empty();
       }
     }

@@ -1,14 +1,31 @@
 // The copying threads of g3a_copy.h against plain copies, with a transfer that
 // moves a slot's bytes only when it is awaited (as late as a DMA may), and one
-// that fails part way.
+// that fails part way; and a crew that finds no memory for its threads.
 #include "g3sa_amd/csrc/g3a_copy.h"
 
 #include <cstdio>
 #include <cstdlib>
+#include <new>
 
 using namespace g3a;
 
+static bool no_memory = false;
+void *operator new(size_t n) {
+  void *p = no_memory ? nullptr : std::malloc(n);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
+
 int main() {
+  {
+    CopyCrew none;  // it is asked from C entry points: nothing may be thrown
+    no_memory = true;
+    const bool ready = none.ready();
+    no_memory = false;
+    if (ready) return std::printf("FAIL ready without memory\n"), 1;
+  }
   CopyCrew crew;
   if (!crew.ready()) return 2;
   const size_t chunk = 4096;
