@@ -902,9 +902,14 @@ static int run_extension(g3a_ctx *ctx, int64_t cap, const int64_t *n_dev, int64_
   if (cap > 0) {
     const bool plain = ctx->form == G3A_FORM_PLAIN;
     Work &w = *ctx->w;
-    const int lane_blocks = ctx->arena ? ctx->run_lane_blocks : ctx->n_cu * ctx->lane_blocks_per_cu,
-              wave_blocks = ctx->n_cu * ctx->wave_blocks_per_cu;
+    const int lane_blocks = ctx->arena ? ctx->run_lane_blocks : ctx->n_cu * ctx->lane_blocks_per_cu;
     const bool group_ok = ext_group_opt_ok(ctx->opt);
+    // With scoring that leaves every task of the plain form to the
+    // one-wavefront kernel, each gets a block: 400,000 reads at a mismatch
+    // score of -9 take 40.1 ms, at the 8 blocks a compute unit that do for the
+    // few tasks it has otherwise 97.7, at all that fit 58.0 (the block with the
+    // longest tasks is waited for).
+    const int wave_blocks = plain && !group_ok ? 0 : ctx->n_cu * ctx->wave_blocks_per_cu;
     const ExtArrays v = ext_arrays(w, cap);
     launch_fill_i32(P<int32_t>(w.ext_ctr), 8, 0, s);
     if (timed && plain) HIPCK(hipEventRecord(ctx->kev[3], s));

@@ -177,6 +177,7 @@ void launch_ext_classify(const ExtSideArgs &a, hipStream_t s);
 // packed: plain columns with two strip rows per register (16-bit lanes)
 void launch_ext_lane(const ExtSideArgs &a, int strip_rows, int packed, int n_blocks, hipStream_t s);
 void launch_ext_group(const ExtSideArgs &a, int n_cu, hipStream_t s);
+// n_blocks 0: a block for each task there may be
 void launch_ext_wave(const ExtSideArgs &a, int n_blocks, hipStream_t s);
 void launch_ext_finish(const ExtFinishArgs &a, hipStream_t s);
 void launch_fill_i32(int32_t *p, int n, int32_t v, hipStream_t s);

@@ -1473,7 +1473,7 @@ void launch_ext_group(const ExtSideArgs &a, int n_cu, hipStream_t s) {
   hipLaunchKernelGGL(k, dim3((unsigned)(need < all ? need : all)), dim3(64), 0, s, a);
 }
 void launch_ext_wave(const ExtSideArgs &a, int n_blocks, hipStream_t s) {
-  if (a.n_tasks) hipLaunchKernelGGL(k_ext_wave, dim3(n_blocks), dim3(64), 0, s, a);
+  if (a.n_tasks) hipLaunchKernelGGL(k_ext_wave, dim3(n_blocks ? (unsigned)n_blocks : (unsigned)a.n_tasks), dim3(64), 0, s, a);
 }
 void launch_ext_finish(const ExtFinishArgs &a, hipStream_t s) {
   if (a.n_tasks) hipLaunchKernelGGL(k_ext_finish, dim3(blocks(a.n_tasks, 256)), dim3(256), 0, s, a);
