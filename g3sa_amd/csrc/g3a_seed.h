@@ -1,11 +1,12 @@
 // Seeding of one read by a group of G lanes (16 on the fast path, a whole
 // wavefront for the reads that outgrow it): rounds 1 to 3 of the reference's
-// seeding with the results of smem_round1, reseed_one and reseed_round3
-// (g3a_dev.h), which run them on one thread.
+// seeding (preseedAndFilterV2, bwa/src/seed.cu:25-104 with 454-531; reseedV2,
+// seed.cu:639-913; reseedThirdRound, seed.cu:1143-1190 with 1518-1550), whose
+// results a host check compares with the same rounds on one thread.
 //
-// What bounds seeding is the chain of dependent Occ fetches: each step of a
-// search needs the interval of the step before.  A thread per read leaves
-// the list entries of a backward step (about 6, up to 64) waiting one after
+// What bounds seeding in a small batch is the chain of dependent Occ fetches:
+// each step of a search needs the interval of the step before (a full chip is
+// bound by instructions, see k_seed).  A thread per read leaves the list entries of a backward step (about 6, up to 64) waiting one after
 // another and most lanes of a load idle (11 of 64).  Here a list entry is a
 // lane: entry e lives in register slot e / G of lane e % G, ends further
 // right as e grows (longest match last), and a backward step is one pair of
