@@ -521,7 +521,7 @@ def main() -> int:
     log("PCIe-inclusive pass")
     pcie = pcie_inclusive(al, batch, 1)
     mean, kms, work = m["stages_ms"], m["kernel_ms"], m["work"]
-    # dominant kernel and its roofline (k_seed: HBM; extension: integer VALU)
+    # dominant kernel and its roofline (k_seed priced against HBM; extension: integer VALU)
     ext_ms = kms["ext_lane"] + kms["ext_wave"]
     # algorithmic bytes of k_seed: each FM step reads the Occ lines of rows
     # k-1 and k+s-1: two 16-byte lines below 2^32 text rows (two 32-byte

@@ -536,13 +536,9 @@ int g3a_device_alloc_sibling(g3a_ctx *src, int max_reads, int64_t max_bases, g3a
   return G3A_OK;
 }
 
-// Workspace of each stage, grown to the batch's sizes (the same calls size it
-// at set-up from max_reads, so that a first batch of typical shape finds it
-// allocated).
-// Grids of a call on n reads: the resident maxima for g3a_bwa_align; for the
-// allocation-free call no more seeding threads than reads, and smaller
-// traceback and extension grids, so that their per-thread pools fit the
-// scratch array.
+// Grids of a call: the resident maxima for g3a_bwa_align; for the
+// allocation-free call smaller traceback and lane-engine grids and slow-path
+// chunks, so that their pools fit the scratch array.
 static void set_grids(g3a_ctx *ctx, bool noalloc) {
   if (!ctx->tb_threads) ctx->tb_threads = traceback_grid_threads(ctx->n_cu);
   ctx->run_tb_threads = ctx->tb_threads;
@@ -557,6 +553,9 @@ static void set_grids(g3a_ctx *ctx, bool noalloc) {
 
 static int alloc_fail(const g3a_ctx *ctx) { return ctx->arena ? G3A_E_ARG : G3A_E_HIP; }
 
+// Workspace of each stage, grown to the batch's sizes (the same calls size it
+// at set-up from max_reads, so that a first batch of typical shape finds it
+// allocated).
 static int alloc_reads(g3a_ctx *ctx, int n) {
   if (ensure(ctx, ctx->w->n_intv, (size_t)n * 4 + 4) || ensure(ctx, ctx->w->n_seed, (size_t)n * 8 + 8) ||
       ensure(ctx, ctx->w->slow, (size_t)n * 4 + 4) || ensure(ctx, ctx->w->intv_base, (size_t)n * 8 + 8) ||

@@ -10,12 +10,16 @@
 
 namespace g3a {
 
-// What bounds it: Occ lines at random places of the table (two of 16 bytes a
-// step, each a 64-byte sector of the cache or of memory) once the chip is full
-// of searches, and the chain of steps of one read in a small batch.  Before, a
-// thread per read; now, at 16 lanes a read (150 bp, 1% substitutions,
-// 100 Mbp): 250,000 reads 4.6 -> 3.0 ms, 200 reads 2.96 -> 0.19 ms; in the
-// wide layout 10.5 -> 3.6 ms; 1,000,000 reads on 1 Gbp 27.5 -> 16.0 ms.
+// What bounds it once the chip is full of searches is integer VALU issue (19
+// instructions a step, 89% of the cycles), with loads pending on the L1 behind
+// it most of the time (two 16-byte Occ lines a step at random places, 0.59 of
+// them from memory at 1 Gbp: 2.1 TB/s); in a small batch the chain of steps of
+// one read.  Before, a thread per read; now, at 16 lanes a read (150 bp, 1%
+// substitutions, 100 Mbp): 250,000 reads 4.6 -> 3.0 ms, 200 reads 2.96 -> 0.20
+// ms; in the wide layout 10.5 -> 3.6 ms; on 1 Gbp 1,000,000 reads 27.5 -> 16.0
+// ms, 10,000,000 190 -> 143 ms.  The learned form takes 14% fewer steps but is
+// no faster (10,000,000 reads 176 -> 152 ms): a model lookup is a chain of
+// dependent loads that one lane of a group waits for.
 // Persistent grid: each group of kSeedLanes lanes takes the next read from a
 // device counter (one atomic per wavefront and turn), so that a group held up
 // by a long read takes fewer.  The superblock counts (narrow: 16 B per 2^21
@@ -146,7 +150,9 @@ void launch_seed(const SeedArgs &a, int n_cu, int blocks_per_cu, int block, hipS
   if (!a.n_reads) return;
   // a batch that leaves compute units idle in blocks of this size runs in
   // smaller ones (200 reads fill 4 blocks of 1024 threads, or 50 of one
-  // wavefront, each on a compute unit of its own)
+  // wavefront, each on a compute unit of its own); blocks_per_cu holds for them
+  // too, so just below 1024, 2048, ... reads a block a compute unit holds half
+  // the reads and they take two turns
   const int64_t threads = (int64_t)a.n_reads * kSeedLanes;
   while (block > 64 && threads < (int64_t)n_cu * block) block = block / 2 / 64 * 64 > 64 ? block / 2 / 64 * 64 : 64;
   const bool narrow = seed_narrow(a.idx);

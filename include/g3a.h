@@ -170,7 +170,9 @@ int g3a_align_batch(g3a_ctx *ctx, int n_reads, const uint8_t *seq, const int32_t
 void g3a_batch_out_free(g3a_batch_out *out);
 /* Stage times (ms: seed, sa, chain, extend, traceback, total) and work
  * counters (seeds, tasks, extension cells, FM steps, slow-path reads,
- * alignments) of the last g3a_bwa_align, without copying its output.  No
+ * alignments) of the last g3a_bwa_align, without copying its output.  The cells
+ * are those of the reference's cell set; the lane engine leaves out the strips
+ * that it prunes.  No
  * reference counterpart: the reference's per-stage timers are the
  * CUDA-event tprof table (bwa/src/bwamem.cu:31-49). */
 int g3a_last_stats(const g3a_ctx *ctx, float ms[6], int64_t work[6]);

@@ -196,9 +196,9 @@ def test_empty_batch(ds_c1):
 
 
 def test_autotune_keeps_output(ds_c1, oracle):
-    """The autotuners rerun the extension stage under every tile shape and the
-    whole batch under every seeding grid and order; the batch's output and
-    every later batch stay identical to the oracle."""
+    """The autotuners rerun the extension stage on the lane engine under every
+    tile shape, and the whole batch under every seeding grid and order; the
+    batch's output and every later batch stay identical to the oracle."""
     names, seq, off, _ = g3sa_amd.read_fastq(str(ds_c1.reads["c3"]), limit=2000)
     idx = oracle.load(ds_c1.prefix)
     try:
@@ -291,9 +291,9 @@ def _tandem_dataset(tmp_path):
 
 
 def test_slow_seeding_path_parity(built, oracle, tmp_path):
-    """Reads inside long tandem repeats grow their LEP lists past the fast
-    seeding path's capacity and are seeded again on the slow path (LDS lists
-    of 400 entries); the output still equals the oracle's."""
+    """Reads inside long tandem repeats outgrow the 64 entries of a 16-lane group
+    (or its 64 intervals) and are seeded again on the slow path, by a wavefront
+    each with 320 entries; the output still equals the oracle's."""
     from types import SimpleNamespace
     prefix, seq, off = _tandem_dataset(tmp_path)
     got, _ = run_both(SimpleNamespace(prefix=prefix), oracle, seq, off, "tandem-repeats")
@@ -313,8 +313,8 @@ def test_slow_seeding_path_parity(built, oracle, tmp_path):
 @pytest.mark.parametrize("which", ["c1", "c3", "rep"])
 def test_wide_layout_parity(ds_c1, ds_rep, oracle, which):
     """The layout of texts of 2^32 rows or more (32-byte Occ lines, 64-bit
-    intervals, no 12-mer table) on texts small enough for the oracle: the
-    seeding, SA lookup and the rest of the path that a 3.1 Gbp index takes,
+    intervals, a 12-mer table of 64-bit fields) on texts small enough for the
+    oracle: the seeding, SA lookup and the rest of the path that a 3.1 Gbp index takes,
     against the oracle in the plain and batched forms."""
     ds = ds_rep if which == "rep" else ds_c1
     fq = ds.reads["main" if which != "c3" else "c3"]
@@ -326,8 +326,8 @@ def test_wide_layout_parity(ds_c1, ds_rep, oracle, which):
 def test_wide_band_global_alignment_parity(built, oracle, tmp_path):
     """Reads of 250 bases carrying one 15-60 base insertion or deletion: their
     global alignments have bands of 2w+1 from about 40 up to 127 columns,
-    computed by the one-wavefront DP (one and two columns per lane) and
-    walked per thread; the CIGARs must equal the oracle's."""
+    computed and walked by a wavefront each (one and two columns per lane); the
+    CIGARs must equal the oracle's."""
     from types import SimpleNamespace
     rng = np.random.default_rng(23)
     L = 300_000
@@ -426,8 +426,8 @@ def _oracle_compat(ds, fq, tmp_path):
 @pytest.mark.parametrize("which", ["rep", "tandem"])
 def test_chain_tiers_equal_serial(ds_rep, tmp_path, which):
     """Chaining by the tiers (a thread per read of at most 16 seeds, a
-    wavefront per read of at most 128, the B-tree code on one lane above)
-    equals the B-tree code for every read, field by field, in the learned and
+    wavefront per read of at most 128, the B-tree on a wavefront above) equals
+    the B-tree code on one thread for every read, field by field, in the learned and
     the FM-index forms, on repeat-rich references whose reads reach every
     tier."""
     if which == "rep":
