@@ -151,8 +151,8 @@ void launch_seed(const SeedArgs &a, int n_cu, int blocks_per_cu, int block, hipS
   // a batch that leaves compute units idle in blocks of this size runs in
   // smaller ones (200 reads fill 4 blocks of 1024 threads, or 50 of one
   // wavefront, each on a compute unit of its own); blocks_per_cu holds for them
-  // too, so just below 1024, 2048, ... reads a block a compute unit holds half
-  // the reads and they take two turns
+  // too, so just below 2048, 4096, ... 16,384 reads (on 256 compute units) half
+  // as many groups as reads are in flight and they take two turns
   const int64_t threads = (int64_t)a.n_reads * kSeedLanes;
   while (block > 64 && threads < (int64_t)n_cu * block) block = block / 2 / 64 * 64 > 64 ? block / 2 / 64 * 64 : 64;
   const bool narrow = seed_narrow(a.idx);
