@@ -1570,3 +1570,7 @@ G3A_HD void trace_and_finalize(const DevIndex &x, const Opt &o, const uint8_t *r
 }
 
 }  // namespace g3a
+
+#if !defined(__HIPCC__)
+#include "g3a_seed_rounds.h"  // for the checks that run on the host
+#endif

@@ -1,8 +1,8 @@
 // The three seeding rounds on one thread, as the reference states them: what
-// the group search of g3a_seed.h is checked against.  Host checks only; no
+// the group search of g3a_seed.h is checked against.  Host builds only; no
 // kernel runs this code.
 #pragma once
-#include "g3sa_amd/csrc/g3a_dev.h"
+#include "g3a_dev.h"
 
 namespace g3a {
 

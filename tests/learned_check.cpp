@@ -17,7 +17,6 @@
 #include "g3sa_amd/csrc/g3a_index.h"
 #include "g3sa_amd/csrc/g3a_layout.h"
 #include "g3sa_amd/csrc/g3a_learned_fit.h"
-#include "tests/seed_rounds.h"
 
 #include <algorithm>
 #include <cstdio>

@@ -1,7 +1,7 @@
 // The group seeding of g3a_seed.h on the host: its lanes run as fibers that
 // meet at each cross-lane operation, and its intervals (k, s, m, n) of every
 // read must equal those of the one-thread code (smem_round1, reseed_one,
-// reseed_round3 of seed_rounds.h).
+// reseed_round3 of g3a_seed_rounds.h).
 //   seed_group_check PREFIX READS [MIN_SEED_LEN]
 // Groups of 16 lanes with 64 entries (the fast path, which may give a read
 // up) and of 64 lanes with 320 (which may not), in the narrow and the wide
@@ -13,7 +13,6 @@
 #include "g3sa_amd/csrc/g3a_layout.h"
 #include "g3sa_amd/csrc/g3a_seed.h"
 #include "tests/fibers.h"
-#include "tests/seed_rounds.h"
 
 #include <cstdio>
 #include <cstdlib>
